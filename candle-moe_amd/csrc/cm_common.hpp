@@ -55,6 +55,30 @@ template <int DT> __device__ __forceinline__ uint32_t pack2(float a, float b) {
     }
 }
 
+// f32 values as their three bf16 parts x = h + m + l (each rounded to
+// nearest even, the differences exact: the parts hold all 24 significand
+// bits), packed in pairs, a low. Non-finite values, and magnitudes that round
+// to a bf16 infinity, give non-finite parts.
+__device__ __forceinline__ void split2(float a, float b, uint32_t& h, uint32_t& m, uint32_t& l) {
+    h = pack2<kBF16>(a, b);
+    a -= __uint_as_float(h << 16);
+    b -= __uint_as_float(h & 0xffff0000u);
+    m = pack2<kBF16>(a, b);
+    a -= __uint_as_float(m << 16);
+    b -= __uint_as_float(m & 0xffff0000u);
+    l = pack2<kBF16>(a, b);
+}
+__device__ __forceinline__ void split8(const float (&v)[8], u32x4& h, u32x4& m, u32x4& l) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        uint32_t x, y, z;
+        split2(v[2 * q], v[2 * q + 1], x, y, z);
+        h[q] = x;
+        m[q] = y;
+        l[q] = z;
+    }
+}
+
 template <int DT> struct Elem;
 template <> struct Elem<kBF16> {
     typedef uint16_t storage;

@@ -154,11 +154,11 @@ constexpr int kTailMinKTiles = 8;  // K tiles per tail split at least (shorter s
 // kW8Gemv (fp8 weights only, moe_gemv_w8.hip): the 32-row tile table, 16
 //   output columns (gate/up) or 32 per workgroup over the whole of K, split
 //   over its 4 waves; operands loaded straight into registers (decode).
-// f32 vector-FMA kernels (moe_gemm_f32.hip): kF32Rows32 (32x128 block tile),
-//   kF32Tile128 (128x128).
+// f32 kernels (moe_gemm_f32.hip, products on the bf16 matrix cores):
+//   kF32Rows32 (32x128 block tile), kF32Tile128 (128x128).
 // The grouping's tile table must be built with the kernel's row tile,
 // tile_rows().
-// kDecGemv (16-bit weights, moe_gemv_dec.hip): decode GEMMs that group the
+// kDecGemv (16-bit, f32 and fp8 weights, moe_gemv_dec.hip): decode GEMMs that group the
 //   pairs themselves (no grouping launch), load weights straight into
 //   registers and split K only across the waves of a workgroup; the down /
 //   fc2 GEMM stores pair rows that the k-row sum adds up.
@@ -210,9 +210,10 @@ inline long long split_grid(long long tiles, const GemmArgs& a) {
     if (a.split_target <= 0) return tiles * a.ksplit;
     return tiles > a.split_target ? tiles : a.split_target;
 }
-// K tile of the LDS-DMA kernels
+// K step of the f32 kernels by tile height, K tile of the LDS-DMA kernels
+constexpr int f32_tile_k(int bm) { return bm == 128 ? 32 : 64; }
 inline int tile_bk(int cfg) {
-    if (is_f32_cfg(cfg)) return 16;
+    if (is_f32_cfg(cfg)) return f32_tile_k(tile_rows(cfg));
     return cfg == kLds128x256o2 ? 32 : 64;
 }
 
@@ -233,7 +234,7 @@ hipError_t launch_w8_gemv(int mode, int dtype, const GemmArgs& a, hipStream_t st
 hipError_t launch_moe_gemm_f32(int mode, int cfg, const GemmArgs& a, hipStream_t stream);
 
 // Decode GEMMs (moe_gemv_dec.hip) over 16-bit weights (API layout or
-// pre-packed) or fp8 codes. Every workgroup groups the P pairs itself (P <=
+// pre-packed), f32 weights (API layout) or fp8 codes. Every workgroup groups the P pairs itself (P <=
 // kDecMaxPairs, E <= kDecMaxE), counts the touched experts U and splits K
 // into ks = min(cap / (U * nblk), ks_lim) slices (at least 1), so that the U
 // * nblk * ks items (expert, column block of 16 * cpl columns, slice) fill
