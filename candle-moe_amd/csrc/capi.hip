@@ -130,6 +130,7 @@ int topk_softmax_impl(const void* g, int gdt, void* w, int wdt, void* idx, void*
 struct Problem {
     int T, H, I, E, k, act, moe_type, dtype;
     bool mfma;
+    bool f32_dec;  // f32 operands the decode kernels can load (16-byte chunks of 8 k)
     bool packed;  // pre-packed K-contiguous 16-bit weights (candle_moe_fused_moe_packed)
     int cfg;  // TileCfg of both GEMMs
     int BM;
@@ -231,6 +232,11 @@ static long long set_tiles_max(const Problem& p) {
     return (p.T + p.BM - 1) / p.BM + (p.nkeys < p.T ? p.nkeys : p.T);
 }
 
+// f32 decode calls: room for the K slices' partials (5 slices of Nomic's fc2
+// and 2 of Qwen3's gate/up at 256 pairs), kept whatever the batch, so that a
+// larger batch never needs a smaller workspace (dec_f32_floor).
+constexpr double kDecPartBytesF32 = 6.0 * 1024 * 1024;
+
 static size_t a256(size_t x) { return (x + 255) & ~(size_t)255; }
 size_t a256_bytes(size_t x) { return a256(x); }
 
@@ -267,7 +273,7 @@ static Layout make_layout(const Problem& p) {
         const size_t nc1 = (size_t)(p.moe_type == kQwen3 ? 2 : 1) * p.I;
         const size_t n1 = p.dec_ks1 > 1 ? (size_t)p.dec_ks1 * p.P * nc1 : 0;  // (ks == 1: rows in the dtype)
         const size_t n2 = (size_t)p.dec_ks2 * p.P * p.H;
-        o += a256(std::max(n1, n2) * 4);
+        o += a256(std::max(std::max(n1, n2) * 4, p.dtype == kF32 ? (size_t)kDecPartBytesF32 : 0));
     } else if (!p.set_path) {
         o += p.rows_path ? a256((size_t)p.P * p.H * es) : a256((size_t)p.T * p.H * 4);
     }
@@ -301,11 +307,17 @@ static Layout make_layout(const Problem& p) {
 // (Their waves' K ranges are whole rounds of 4 steps of 32, which may run
 // up to 512 past K: the weight offsets stay below 2^31 with that margin.)
 static bool dec_gemv_fits(const Problem& p) {
-    const long long lim = 0x7fffff00LL;
-    return p.mfma && p.P <= kDecMaxPairs && p.E <= kDecMaxE && (long long)p.T * p.H * 2 < lim &&
-           p.P * p.I * 2 < lim && p.P * p.H * 2 < lim && (long long)(p.H + 1024) * p.I * 2 < lim &&
-           (long long)(p.I + 1024) * p.H * 2 < lim;
+    const long long lim = 0x7fffff00LL, es = p.dtype == kF32 ? 4 : 2;
+    return (p.mfma || p.f32_dec) && p.P <= kDecMaxPairs && p.E <= kDecMaxE && (long long)p.T * p.H * es < lim &&
+           p.P * p.I * es < lim && p.P * p.H * es < lim && (long long)(p.H + 1024) * p.I * es < lim &&
+           (long long)(p.I + 1024) * p.H * es < lim;
 }
+
+// Workspace of the largest f32 decode call of this layer (dtype, H, I, E, k):
+// the f32 tile kernels that larger batches take need less in places, and a
+// workspace grown (or sized by the caller) for a batch has to do for every
+// smaller one, also under graph capture, where it cannot grow.
+static size_t dec_f32_floor(const Problem& p);
 
 // Most K slices of a decode GEMM over N columns and K (the kernels choose
 // the slices from the experts a batch touches, up to this): cold weights
@@ -319,10 +331,10 @@ static bool dec_gemv_fits(const Problem& p) {
 constexpr int kDecMinSteps = 1;
 constexpr double kDecPartBytes = 16.0 * 1024 * 1024;
 constexpr double kDecSliceBytes = 128.0 * 1024 * 1024;
-static int dec_slices(long long P, int N, int K, int kp, int nc_mult) {
+static int dec_slices(long long P, int N, int K, int kp, int nc_mult, double part_bytes) {
     long long ks = cdiv(K, 32) / (kp * kDecMinSteps);
     ks = std::min<long long>(ks, kDecMaxSlices);
-    ks = std::min<long long>(ks, (long long)(kDecPartBytes / ((double)std::max<long long>(P, 1) * N * nc_mult * 4)));
+    ks = std::min<long long>(ks, (long long)(part_bytes / ((double)std::max<long long>(P, 1) * N * nc_mult * 4)));
     return (int)std::max<long long>(ks, 1);
 }
 // Workgroups of one round of the decode kernels: two per CU.
@@ -342,9 +354,10 @@ constexpr long long kDecDefaultPairs = 256;
 // handles any alignment).
 // fp8: fp8 weights (candle_moe_fused_moe_fp8): the 32-row kernel for decode
 // batches, the 8-wave 256x256 kernel beyond, on the pair path.
+// f32_dec: f32 calls may take the decode kernels.
 static int check_problem(int T, int H, int I, int E, int k, int act, uint32_t moe_type, uint32_t dtype,
                          Problem& p, bool aligned16 = true, bool out16 = true, bool fp8 = false,
-                         bool packed = false) {
+                         bool packed = false, bool f32_dec = true) {
     if (T < 0) return set_error(CANDLE_MOE_ERR_INVALID, "fused_moe: num_tokens must be >= 0 (got %d)", T);
     if (H < 1 || I < 1)
         return set_error(CANDLE_MOE_ERR_INVALID, "fused_moe: hidden_dim and intermediate_dim must be >= 1 (got %d, %d)", H, I);
@@ -389,12 +402,22 @@ static int check_problem(int T, int H, int I, int E, int k, int act, uint32_t mo
     int policy = g_tile_policy == kW8Gemv ? 0 : g_tile_policy;
     if (packed && policy && !is_lds_cfg(policy) && policy != kDecGemv) policy = 0;
     p.cfg = !p.mfma ? kTileSimt : (policy ? policy : kLds256w8);
-    // f32: the tiled vector-FMA kernel (32-row tile with K splits for decode,
-    // 128-row tile otherwise) wherever 16-byte loads are possible
+    // f32: the split-bf16 kernels (decode kernels, 32-row or 128-row tiles)
+    // wherever 16-byte loads are possible
     const bool f32_tiled = p.dtype == kF32 && H % 4 == 0 && I % 4 == 0 && aligned16;
+    p.f32_dec = f32_dec && p.dtype == kF32 && H % 8 == 0 && I % 8 == 0 && aligned16;
     if (f32_tiled) {
-        p.cfg = (P <= 32 * touched) ? kF32Rows32 : kF32Tile128;
-        if (policy == kF32Rows32 || policy == kF32Tile128) p.cfg = policy;
+        // 32-row tiles up to 64 rows per touched expert (steps, 32-row against
+        // 128-row tiles: Nomic T=129 / 256 118 / 109 against 141 / 153 us,
+        // Qwen3 T=140 / 200 239 / 220 against 306 / 309 us; beyond, Qwen3
+        // T=300 388 against 332 us); the decode kernels, which read the
+        // weights once per 32 rows without the grouping launch and the LDS
+        // staging, up to 32 rows per expert and the 16-bit path's 256 pairs
+        // (Nomic T=64 / 128 54 / 83 against 86 / 118 us, Qwen3 T=8 / 100 118 /
+        // 175 against 153 / 206 us; T=128 237 against 229 us)
+        p.cfg = (P <= 64 * touched) ? kF32Rows32 : kF32Tile128;
+        if (P <= 32 * touched && P <= kDecDefaultPairs && dec_gemv_fits(p)) p.cfg = kDecGemv;
+        if (policy == kF32Rows32 || policy == kF32Tile128 || (policy == kDecGemv && dec_gemv_fits(p))) p.cfg = policy;
     } else if (!p.mfma || is_f32_cfg(p.cfg)) {
         p.cfg = kTileSimt;
     }
@@ -586,11 +609,24 @@ static int check_problem(int T, int H, int I, int E, int k, int act, uint32_t mo
         // pairs anyway, ran 1-3 us faster unsliced on every shape.
         const bool q3 = p.moe_type == kQwen3;
         const long long groups = std::min<long long>(P, E);
-        const double wbytes = (double)groups * (q3 ? 2 : 1) * H * I * (fp8 ? 1 : 2);
-        if (groups * cdiv(I, 128) < 256 && wbytes >= kDecSliceBytes)
-            p.dec_ks1 = dec_slices(P, I, H, q3 ? 2 : 4, q3 ? 2 : 1);
+        const double wbytes = (double)groups * (q3 ? 2 : 1) * H * I * (fp8 ? 1 : p.dtype == kF32 ? 4 : 2);
+        // f32 (blocks of 64 columns): slices for the down / fc2 GEMM too where
+        // its items would leave CUs idle (Nomic's fc2 has 96 of them)
+        const int cols = p.dtype == kF32 ? 64 : 128;
+        const double part = p.dtype == kF32 ? kDecPartBytesF32 : kDecPartBytes;
+        if (groups * cdiv(I, cols) < 256 && wbytes >= kDecSliceBytes)
+            p.dec_ks1 = dec_slices(P, I, H, q3 ? 2 : 4, q3 ? 2 : 1, part);
+        if (p.dtype == kF32 && groups * cdiv(H, cols) < 256) p.dec_ks2 = dec_slices(P, H, I, 4, 1, part);
     }
     return CANDLE_MOE_OK;
+}
+
+static size_t dec_f32_floor(const Problem& p) {
+    if (!p.f32_dec || p.cfg == kDecGemv) return 0;
+    Problem q;
+    const int T = (int)std::min<long long>(p.T, std::max<long long>(std::min<long long>(kDecDefaultPairs, 32LL * p.E) / p.k, 1));
+    if (check_problem(T, p.H, p.I, p.E, p.k, p.act, (uint32_t)p.moe_type, (uint32_t)p.dtype, q)) return 0;
+    return q.cfg == kDecGemv ? make_layout(q).total : 0;
 }
 
 // fp8 expert weights of candle_moe_fused_moe_fp8 (codes [E][N][K], scales [E][N])
@@ -615,7 +651,9 @@ struct Fp8Weights {
 // [N,K] weights (16-byte loads of 16 columns whatever the block): 8, 6, 4, 3
 // or 2 (blocks of 48 and 96 columns put Qwen3's 1536 and Nomic's 3072
 // columns of 8 experts into 256 items).
-static int dec_cpl(long long groups, int N, bool trans, int ks_lim) {
+// f32: 4 columns (the same 16 bytes per lane and k-row; slices even out the items).
+static int dec_cpl(long long groups, int N, bool trans, int ks_lim, bool f32) {
+    if (f32) return 4;
     if (ks_lim > 1) return 8;
     const double cus = 8.0 * std::max(cus_per_xcd(), 32);
     static const int kTrans[] = {8, 4}, kNK[] = {8, 6, 4, 3, 2};
@@ -662,12 +700,13 @@ static int run_moe_dec(const Problem& p, const void* x, const void* gate, const 
         d.scale0 = f8->gate_scale;
         d.scale1 = f8->up_scale;
     }
-    d.a_bytes = (long long)p.T * p.H * 2;
+    const int es = p.dtype == kF32 ? 4 : 2;
+    d.a_bytes = (long long)p.T * p.H * es;
     d.max_groups = (int)std::min<long long>(p.P, p.E);
     d.rows_max = (int)std::min<long long>(p.P, p.T);
     d.cap = dec_cap();
     d.ks_lim = p.dec_ks1;
-    d.cpl = dec_cpl(d.max_groups, p.I, !p.packed && !f8, d.ks_lim);
+    d.cpl = dec_cpl(d.max_groups, p.I, !p.packed && !f8, d.ks_lim, p.dtype == kF32);
     d.nblk = cdiv(p.I, 16 * d.cpl);
     const int mode1 = qwen3 ? kGateUp : kFc1;
     hipError_t e;
@@ -701,14 +740,14 @@ static int run_moe_dec(const Problem& p, const void* x, const void* gate, const 
     d2.K = p.I;
     d2.N = p.H;
     d2.ldb = (qwen3 && !p.packed && !f8) ? p.H : p.I;  // down [E][I][H] (packed / fp8 [E][H][I]); fc2 [E][H][I]
-    d2.a_bytes = p.P * p.I * 2;
+    d2.a_bytes = p.P * p.I * es;
     d2.ks_lim = p.dec_ks2;
     // fp8 column scales: multiplied in by the GEMM when it is not K-sliced
     // (its partials are then whole sums), else by the finishing launch
     const float* s2 = f8 ? (qwen3 ? f8->down_scale : f8->up_scale) : nullptr;
     d2.scale0 = d2.ks_lim == 1 ? s2 : nullptr;
     d2.scale1 = nullptr;
-    d2.cpl = dec_cpl(d.max_groups, p.H, qwen3 && !p.packed && !f8, d2.ks_lim);
+    d2.cpl = dec_cpl(d.max_groups, p.H, qwen3 && !p.packed && !f8, d2.ks_lim, p.dtype == kF32);
     d2.nblk = cdiv(p.H, 16 * d2.cpl);
     {
         ProfScope ps(kSlotGemm2, s);
@@ -965,17 +1004,21 @@ static std::vector<OwnedWs> g_ws;
 // (err = hipErrorStreamCaptureUnsupported): hipMallocAsync there would add an
 // allocation node to the caller's graph, memory the graph owns and releases
 // when it is destroyed, while this table would keep handing it out.
-static OwnedWs* owned_ws_locked(int dev, hipStream_t s, size_t need, hipError_t& err) {
+// reserve: bytes wanted beyond need for later calls, not insisted on in a
+// capture.
+static OwnedWs* owned_ws_locked(int dev, hipStream_t s, size_t need, hipError_t& err, size_t reserve = 0) {
     err = hipSuccess;
     OwnedWs* w = nullptr;
     for (auto& e : g_ws)
         if (e.device == dev && e.stream == s) w = &e;
-    if (w && w->bytes >= need) return w;
+    if (w && w->bytes >= std::max(need, reserve)) return w;
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone) {
+        if (w && w->bytes >= need) return w;
         err = hipErrorStreamCaptureUnsupported;
         return nullptr;
     }
+    need = std::max(need, reserve);
     // grow by at least 1.5x and to whole MiB, so that a slowly growing T
     // does not reallocate on every call
     size_t want = need + need / 2;
@@ -1056,7 +1099,7 @@ int fused_moe_impl(const void* x, const void* gate, const void* up, const void* 
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return hip_fail(e, "fused_moe: hipGetDevice");
     std::lock_guard<std::mutex> lk(g_ws_mu);
-    OwnedWs* w = owned_ws_locked(dev, s, L.total, e);
+    OwnedWs* w = owned_ws_locked(dev, s, L.total, e, dec_f32_floor(p));
     if (!w) return ws_fail("fused_moe", L.total, e);
     return run_moe(p, x, gate, up, down, reinterpret_cast<const float*>(rw), reinterpret_cast<const uint32_t*>(idx),
                    out, overwrite, reinterpret_cast<char*>(w->ptr), s, f8, true);
@@ -1105,7 +1148,13 @@ int fused_moe_noalloc_impl(const void* x, const void* gate, const void* up, cons
     rc = check_ptrs(p, x, gate, up, down, rw, idx, out);
     if (rc) return rc;
     if (T == 0) return CANDLE_MOE_OK;
-    const Layout L = make_layout(p);
+    Layout L = make_layout(p);
+    if (L.total > kNoAllocScratchBytes && p.cfg == kDecGemv && p.dtype == kF32) {
+        // (the f32 tile kernels, which keep no partials by pair, may still fit)
+        rc = check_problem(T, H, I, E, k, act, moe_type, dtype, p, aligned16, a16(out), false, false, false);
+        if (rc) return rc;
+        L = make_layout(p);
+    }
     if (L.total > kNoAllocScratchBytes)
         return set_error(CANDLE_MOE_ERR_WORKSPACE,
                          "fused_moe_noalloc: this call needs %zu bytes of scratch; the library holds %zu per device "
@@ -1134,7 +1183,7 @@ size_t fused_moe_ws_size(int T, int H, int I, int E, int k, uint32_t dtype) {
         for (int al = 0; al < 2; ++al) {
             Problem p;
             if (check_problem(T, H, I, E, k, 0, mt, dtype, p, al != 0)) return 0;
-            most = std::max(most, make_layout(p).total);
+            most = std::max(most, std::max(make_layout(p).total, dec_f32_floor(p)));
         }
     return most;
 }

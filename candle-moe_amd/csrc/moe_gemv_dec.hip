@@ -1,5 +1,6 @@
-// Decode GEMMs over 16-bit expert weights (API layout or pre-packed) or fp8
-// codes (gfx950), with no grouping launch and no LDS staging of the weights.
+// Decode GEMMs over 16-bit expert weights (API layout or pre-packed), fp8
+// codes or f32 weights (gfx950), with no grouping launch and no LDS staging of
+// the weights.
 //
 // At decode sizes the work is the weight stream and the fixed latency around
 // it. The 32-row tile kernel needs the grouping's tile table (a launch and
@@ -65,9 +66,9 @@ constexpr int kDvStep = 32;  // K per step (one MFMA deep)
 // steps in flight per wave: 4, or 2 for 6 or 8 columns per lane, so that a
 // wave stays within 256 registers and two workgroups share a CU; halved where
 // each column takes WCH = 2 chunks of 16 bytes per step (the same bytes in
-// flight)
-template <int CPL, int WCH = 1>
-constexpr int dec_ring() { return (CPL >= 6 ? 2 : 4) / WCH; }
+// flight). f32: twice the bytes per weight, so 2 steps from 3 columns on.
+template <int CPL, int WCH = 1, bool F32 = false>
+constexpr int dec_ring() { return F32 ? (CPL >= 3 ? 2 : 4) : (CPL >= 6 ? 2 : 4) / WCH; }
 
 // Operand j of a transposed 8 x CPL block: r[t] holds k-row t of CPL
 // consecutive columns (pairs of 16-bit values, low half first); the result
@@ -211,14 +212,19 @@ __device__ __forceinline__ void finish_pair4(const DecFinish& f, int ks, long lo
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const float s0 = W8 ? f.scale0[(long long)e * f.N + c + j] : 1.0f;
+            const float y = DT == kF32 ? act_f32(g[j], ACT) : act_t<ACT>(s0 * g[j]);
             if constexpr (DUAL) {
                 const float s1 = W8 ? f.scale1[(long long)e * f.N + c + j] : 1.0f;
-                h[j] = act_t<ACT>(s0 * g[j]) * (s1 * u[j]);
+                h[j] = y * (s1 * u[j]);
             } else {
-                h[j] = act_t<ACT>(s0 * g[j]);
+                h[j] = y;
             }
         }
     });
+    if constexpr (DT == kF32) {
+        *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(f.out) + p * f.N + c) = f32x4{h[0], h[1], h[2], h[3]};
+        return;
+    }
     *reinterpret_cast<u32x2*>(reinterpret_cast<uint16_t*>(f.out) + p * f.N + c) =
         u32x2{pack2<DT>(h[0], h[1]), pack2<DT>(h[2], h[3])};
 }
@@ -227,8 +233,9 @@ __device__ __forceinline__ void finish_pair4(const DecFinish& f, int ks, long lo
 template <int DT, bool W8, int KSM, int KM>
 __device__ __forceinline__ void finish_token4(const DecFinish& f, int ks, long long t, int c) {
     const long long stride = (long long)f.P * f.N;
-    uint16_t* orow = reinterpret_cast<uint16_t*>(f.out) + t * f.N + c;
-    const bool al8 = (reinterpret_cast<uintptr_t>(f.out) & 7u) == 0;  // else 2-byte accesses
+    typedef typename Elem<DT>::storage ST;
+    ST* orow = reinterpret_cast<ST*>(f.out) + t * f.N + c;
+    const bool al = (reinterpret_cast<uintptr_t>(f.out) & (4 * sizeof(ST) - 1)) == 0;  // else one element at a time
     float acc[4] = {0.f, 0.f, 0.f, 0.f};
     if (!f.overwrite) {
 #pragma unroll
@@ -260,12 +267,22 @@ __device__ __forceinline__ void finish_token4(const DecFinish& f, int ks, long l
             }
         }
     }
-    const u32x2 o = {pack2<DT>(acc[0], acc[1]), pack2<DT>(acc[2], acc[3])};
-    if (al8) {
-        *reinterpret_cast<u32x2*>(orow) = o;
-    } else {
+    if constexpr (DT == kF32) {
+        if (al) {
+            *reinterpret_cast<f32x4*>(orow) = f32x4{acc[0], acc[1], acc[2], acc[3]};
+        } else {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) orow[j] = (uint16_t)((o[j >> 1] >> (16 * (j & 1))) & 0xffffu);
+            for (int j = 0; j < 4; ++j) orow[j] = acc[j];
+        }
+        return;
+    } else {
+        const u32x2 o = {pack2<DT>(acc[0], acc[1]), pack2<DT>(acc[2], acc[3])};
+        if (al) {
+            *reinterpret_cast<u32x2*>(orow) = o;
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) orow[j] = (uint16_t)((o[j >> 1] >> (16 * (j & 1))) & 0xffffu);
+        }
     }
 }
 
@@ -288,12 +305,20 @@ __global__ __launch_bounds__(64 * kDvWaves, 2) void moe_dec_gemv(DecArgs a) {
     // T=16 bf16 fc2 15.4 -> 13.9 us). The other pre-packed GEMMs keep one
     // chunk: the same k per MFMA as on the API layout, hence the same sums
     // bit for bit.
+    // f32 weights: every value is split into three bf16 parts in registers and
+    // a product is the sum of six part MFMAs (moe_gemm_f32.hip says why and at
+    // what error). [K,N]: 8 loads of CPL f32 per lane and step, as the 16-bit
+    // form (whose v_perm transpose the pairwise conversion replaces); [N,K]:
+    // two 16-byte chunks of 4 k, 128 contiguous bytes per column and step.
+    constexpr bool F32 = DT == kF32;
+    static_assert(!F32 || (!W8 && !PK && CPL <= 4), "f32: API layout, at most 4 columns per lane");
     constexpr int WCH = (W8 || MODE == kFc2Rows) ? 2 : 1;
-    constexpr int KSTEP = (W8 ? 64 : kDvStep) * WCH;
-    constexpr int KG = (W8 ? 16 : 8) * WCH;  // k per lane group per step
-    constexpr int KC = W8 ? 16 : 8;         // k per 16-byte weight chunk
-    constexpr int WB = W8 ? 1 : 2;          // bytes per weight
-    constexpr int AH = (W8 ? 2 : 1) * WCH;   // 16-byte A loads per row and step
+    constexpr int KSTEP = F32 ? kDvStep : (W8 ? 64 : kDvStep) * WCH;
+    constexpr int KG = F32 ? 8 : (W8 ? 16 : 8) * WCH;  // k per lane group per step
+    constexpr int KC = F32 ? 8 / WCH : W8 ? 16 : 8;    // k per weight chunk
+    constexpr int WB = F32 ? 4 : W8 ? 1 : 2;           // bytes per weight
+    constexpr int AB = F32 ? 4 : 2;                    // bytes per activation
+    constexpr int AH = F32 ? 2 : (W8 ? 2 : 1) * WCH;   // 16-byte A loads per row and step
     constexpr bool ROWS = (MODE == kDownRows || MODE == kFc2Rows);
     constexpr int NT = 64 * kDvWaves;
     constexpr int WGC = 16 * CPL;                // output columns per workgroup
@@ -345,7 +370,7 @@ __global__ __launch_bounds__(64 * kDvWaves, 2) void moe_dec_gemv(DecArgs a) {
     // whole number of ring rounds (the steps past s_hi load zeros), so that
     // the ring loop needs no guard. The parts depend on K, the slices and the
     // waves only (not on the ring or the column block).
-    constexpr int RING = dec_ring<CPL, WCH>();
+    constexpr int RING = dec_ring<CPL, WCH, F32>();
     const int nks = (K + KSTEP - 1) / KSTEP;
     const int nparts = KP * ks;
     const int per = (nks + nparts - 1) / nparts;
@@ -367,7 +392,7 @@ __global__ __launch_bounds__(64 * kDvWaves, 2) void moe_dec_gemv(DecArgs a) {
     uint32_t wlane[TRANS ? 1 : NB];
 #pragma unroll
     for (int b = 0; b < (TRANS ? 1 : NB); ++b)
-        wlane[b] = ncol[b] < N ? (TRANS ? 8u * (uint32_t)g * ldb2 + 2u * (uint32_t)ncol[0]
+        wlane[b] = ncol[b] < N ? (TRANS ? 8u * (uint32_t)g * ldb2 + (uint32_t)WB * (uint32_t)ncol[0]
                                         : (uint32_t)ncol[b] * ldb2 + (uint32_t)(KG * WB) * (uint32_t)g)
                                : kOob;
 
@@ -375,7 +400,7 @@ __global__ __launch_bounds__(64 * kDvWaves, 2) void moe_dec_gemv(DecArgs a) {
     // [N,K]) and the A rows. Branch-free offsets (a branch, or a select on
     // the step alone, made the compiler wait for every load in flight): a
     // lane's k positions past K read zeros (kOob).
-    constexpr int WDW = TRANS ? CPL / 2 : 4;  // dwords per weight load
+    constexpr int WDW = TRANS ? CPL * WB / 4 : 4;  // dwords per weight load
     uint32_t wv[RING][NLD][WDW];
     u32x4 xv[RING][RB][AH];
     // this lane's k of step s, chunk c, inside the wave's part and K (K is a
@@ -429,13 +454,21 @@ __global__ __launch_bounds__(64 * kDvWaves, 2) void moe_dec_gemv(DecArgs a) {
             const int m = rb * 16 + li;
             const int p = s_rows[c0 + min(m, m_valid - 1)];
             const int src = GATHER ? p / a.k_top : p;
-            abase[rb] = m < m_valid ? ((uint32_t)src * (uint32_t)K + (uint32_t)(KG * g)) * 2u : kOob;
+            abase[rb] = m < m_valid ? ((uint32_t)src * (uint32_t)K + (uint32_t)(KG * g)) * (uint32_t)AB : kOob;
         }
         f32x4 acc[RB][NB];
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
             for (int b = 0; b < NB; ++b) acc[rb][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+        // (f32: the five small part products apart from the large one)
+        f32x4 small[F32 ? RB : 1][F32 ? NB : 1];
+        if constexpr (F32) {
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+                for (int b = 0; b < NB; ++b) small[rb][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
         auto load_a = [&](int i, int st) {
             const int s = s_lo + st;
 #pragma unroll
@@ -445,7 +478,7 @@ __global__ __launch_bounds__(64 * kDvWaves, 2) void moe_dec_gemv(DecArgs a) {
                     // load h holds the k of weight chunk h / (AH / WCH)
                     const bool kok = k_ok(s, h / (AH / WCH));
                     xv[i][rb][h] = __builtin_amdgcn_raw_buffer_load_b128(
-                        rx, kok ? abase[rb] + (uint32_t)(s * KSTEP) * 2u + 16u * h : kOob, 0, 0);
+                        rx, kok ? abase[rb] + (uint32_t)(s * KSTEP * AB) + 16u * h : kOob, 0, 0);
                 }
         };
         auto load = [&](int i, int st) {
@@ -453,9 +486,35 @@ __global__ __launch_bounds__(64 * kDvWaves, 2) void moe_dec_gemv(DecArgs a) {
             load_a(i, st);
         };
         auto compute = [&](int i) {
+            u32x4 ap[F32 ? RB : 1][3];
+            if constexpr (F32) {
+#pragma unroll
+                for (int rb = 0; rb < RB; ++rb) {
+                    const u32x4 x = xv[i][rb][0], y = xv[i][rb][AH - 1];
+                    const float v[8] = {__uint_as_float(x[0]), __uint_as_float(x[1]), __uint_as_float(x[2]),
+                                        __uint_as_float(x[3]), __uint_as_float(y[0]), __uint_as_float(y[1]),
+                                        __uint_as_float(y[2]), __uint_as_float(y[3])};
+                    split8(v, ap[rb][0], ap[rb][1], ap[rb][2]);
+                }
+            }
 #pragma unroll
             for (int b = 0; b < NB; ++b) {
-                if constexpr (W8) {
+                if constexpr (F32) {
+                    float v[8];
+#pragma unroll
+                    for (int t = 0; t < 8; ++t)
+                        v[t] = __uint_as_float(TRANS ? wv[i][t][b % WDW] : wv[i][b * WCH + t / 4][t % 4]);
+                    u32x4 bp[3];
+                    split8(v, bp[0], bp[1], bp[2]);
+                    constexpr int PA[5] = {2, 0, 1, 1, 0}, PB[5] = {0, 2, 1, 0, 1};
+#pragma unroll
+                    for (int q = 0; q < 5; ++q)
+#pragma unroll
+                        for (int rb = 0; rb < RB; ++rb)
+                            small[rb][b] = mfma16<kBF16>(ap[rb][PA[q]], bp[PB[q]], small[rb][b]);
+#pragma unroll
+                    for (int rb = 0; rb < RB; ++rb) acc[rb][b] = mfma16<kBF16>(ap[rb][0], bp[0], acc[rb][b]);
+                } else if constexpr (W8) {
                     // chunk c: codes k0 + KG g + 16c .. +7 and .. +15 of
                     // column b, two operands; A loads 2c and 2c + 1 hold the
                     // same k of the row
@@ -525,6 +584,53 @@ __global__ __launch_bounds__(64 * kDvWaves, 2) void moe_dec_gemv(DecArgs a) {
         }
 #pragma unroll
         for (int i = 0; i < RING; ++i) compute(i);
+
+        if constexpr (F32) {
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+                for (int b = 0; b < NB; ++b)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) acc[rb][b][v] += small[rb][b][v];
+            // blocks with a non-finite sum (infinities, NaN, values whose bf16
+            // part rounds to infinity, overflow) again with f32 FMAs over this
+            // wave's k (an element past the operands reads zero)
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+                bool bad = false;
+#pragma unroll
+                for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) bad |= !__builtin_isfinite(acc[rb][b][v]);
+                if (__builtin_expect(__any(bad), 0)) {
+                    uint32_t arow[RB][4];
+#pragma unroll
+                    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+                        for (int v = 0; v < 4; ++v) {
+                            const int m = rb * 16 + 4 * g + v;
+                            const int p = s_rows[c0 + min(m, m_valid - 1)];
+                            arow[rb][v] = (uint32_t)(GATHER ? p / a.k_top : p) * (uint32_t)K * 4u;
+                            acc[rb][b][v] = 0.f;
+                        }
+                    const int col = min(ncol[b], N - 1);
+                    const int k_hi = min(K, s_hi * KSTEP);
+                    for (int k = s_lo * KSTEP; k < k_hi; ++k) {
+                        const uint32_t wo = TRANS ? (uint32_t)k * ldb2 + 4u * (uint32_t)col
+                                                  : (uint32_t)col * ldb2 + 4u * (uint32_t)k;
+                        const float w = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rw, wo, 0, 0));
+#pragma unroll
+                        for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+                            for (int v = 0; v < 4; ++v) {
+                                const float x = __uint_as_float(
+                                    __builtin_amdgcn_raw_buffer_load_b32(rx, arow[rb][v] + 4u * (uint32_t)k, 0, 0));
+                                acc[rb][b][v] = fmaf(x, w, acc[rb][b][v]);
+                            }
+                    }
+                }
+            }
+        }
 
         // parts to LDS: lane (g, li) holds rows 4g .. 4g+3 of each row block
         // at local column CPL*li + b ([K,N]: CPL consecutive columns, stored
@@ -616,12 +722,20 @@ __global__ __launch_bounds__(64 * kDvWaves, 2) void moe_dec_gemv(DecArgs a) {
                         // (fp8 weights: the column scales on the f32 sums first)
                         const int cc = col + j;
                         const float s0 = W8 ? (cc < N ? a.scale0[(long long)e * N + cc] : 0.0f) : 1.0f;
+                        const float y = F32 ? act_f32(y0[j], ACT) : act_t<ACT>(s0 * y0[j]);
                         if constexpr (DUAL) {
                             const float s1 = W8 ? (cc < N ? a.scale1[(long long)e * N + cc] : 0.0f) : 1.0f;
-                            h[j] = act_t<ACT>(s0 * y0[j]) * (s1 * y1[j]);
+                            h[j] = y * (s1 * y1[j]);
                         } else {
-                            h[j] = act_t<ACT>(s0 * y0[j]);
+                            h[j] = y;
                         }
+                    }
+                    if constexpr (F32) {
+                        // (N and col are multiples of 8: whole chunks)
+                        float* C = reinterpret_cast<float*>(a.C) + (long long)p * N + col;
+                        *reinterpret_cast<f32x4*>(C) = f32x4{h[0], h[1], h[2], h[3]};
+                        *reinterpret_cast<f32x4*>(C + 4) = f32x4{h[4], h[5], h[6], h[7]};
+                        continue;
                     }
                     u32x4 o;
 #pragma unroll
@@ -667,20 +781,26 @@ hipError_t launch_cfg(const DecArgs& a, hipStream_t stream) {
     if (nwg > 0x7fffffffLL) return hipErrorInvalidValue;
     if (a.max_groups <= 0) return hipSuccess;
     const dim3 grid((int)nwg), block(64 * kDvWaves);
-    if (a.w8) {
-        // fp8 codes are [N,K] for every GEMM (Nomic's fc2 runs the down mode)
-        constexpr int M8 = MODE == kFc2Rows ? kDownRows : MODE;
-        hipLaunchKernelGGL((moe_dec_gemv<DT, M8, RB, CPL, false, true>), grid, block, 0, stream, a);
+    if constexpr (DT != kF32) {
+        if (a.w8) {
+            // fp8 codes are [N,K] for every GEMM (Nomic's fc2 runs the down mode)
+            constexpr int M8 = MODE == kFc2Rows ? kDownRows : MODE;
+            hipLaunchKernelGGL((moe_dec_gemv<DT, M8, RB, CPL, false, true>), grid, block, 0, stream, a);
+            return hipGetLastError();
+        }
+    }
+    if constexpr (DT == kF32) {
+        hipLaunchKernelGGL((moe_dec_gemv<DT, MODE, RB, CPL, false, false>), grid, block, 0, stream, a);
         return hipGetLastError();
     }
     // (Nomic's fc2 is [N,K] either way: no packed instance)
-    if constexpr (MODE != kFc2Rows) {
+    if constexpr (MODE != kFc2Rows && DT != kF32) {
         if (a.packed) {
             hipLaunchKernelGGL((moe_dec_gemv<DT, MODE, RB, CPL, true, false>), grid, block, 0, stream, a);
             return hipGetLastError();
         }
     }
-    if constexpr (MODE == kFc2Rows || (CPL != 3 && CPL != 6)) {
+    if constexpr (DT != kF32 && (MODE == kFc2Rows || (CPL != 3 && CPL != 6))) {
         hipLaunchKernelGGL((moe_dec_gemv<DT, MODE, RB, CPL, false, false>), grid, block, 0, stream, a);
         return hipGetLastError();
     }
@@ -690,11 +810,22 @@ hipError_t launch_cfg(const DecArgs& a, hipStream_t stream) {
 template <int DT, int MODE>
 hipError_t launch_mode(const DecArgs& a, hipStream_t stream) {
     const bool rb2 = a.rows_max > 16;
+    if constexpr (DT == kF32) {
+        // f32: 4 columns per lane ([N,K] also 3 and 2)
+        if (a.w8 || a.packed) return hipErrorInvalidValue;
+        if constexpr (MODE == kFc2Rows) {
+            if (a.cpl == 2) return rb2 ? launch_cfg<DT, MODE, 2, 2>(a, stream) : launch_cfg<DT, MODE, 1, 2>(a, stream);
+            if (a.cpl == 3) return rb2 ? launch_cfg<DT, MODE, 2, 3>(a, stream) : launch_cfg<DT, MODE, 1, 3>(a, stream);
+        }
+        if (a.cpl != 4) return hipErrorInvalidValue;
+        return rb2 ? launch_cfg<DT, MODE, 2, 4>(a, stream) : launch_cfg<DT, MODE, 1, 4>(a, stream);
+    } else {
     if (a.cpl == 2) return rb2 ? launch_cfg<DT, MODE, 2, 2>(a, stream) : launch_cfg<DT, MODE, 1, 2>(a, stream);
     if (a.cpl == 3) return rb2 ? launch_cfg<DT, MODE, 2, 3>(a, stream) : launch_cfg<DT, MODE, 1, 3>(a, stream);
     if (a.cpl == 6) return rb2 ? launch_cfg<DT, MODE, 2, 6>(a, stream) : launch_cfg<DT, MODE, 1, 6>(a, stream);
     if (a.cpl == 4) return rb2 ? launch_cfg<DT, MODE, 2, 4>(a, stream) : launch_cfg<DT, MODE, 1, 4>(a, stream);
     return rb2 ? launch_cfg<DT, MODE, 2, 8>(a, stream) : launch_cfg<DT, MODE, 1, 8>(a, stream);
+    }
 }
 
 template <int DT>
@@ -719,6 +850,7 @@ hipError_t launch_dec_gemv(int mode, int dtype, const DecArgs& a, hipStream_t st
         return hipErrorInvalidValue;
     if (dtype == kBF16) return launch_dt<kBF16>(mode, a, stream);
     if (dtype == kF16) return launch_dt<kF16>(mode, a, stream);
+    if (dtype == kF32) return launch_dt<kF32>(mode, a, stream);
     return hipErrorInvalidValue;
 }
 
@@ -751,7 +883,10 @@ hipError_t finish_mode(const DecFinish& f, hipStream_t stream) {
     if (n <= 0) return hipSuccess;
     if ((n + 63) / 64 > 0x7fffffffLL) return hipErrorInvalidValue;
     const dim3 grid((unsigned)((n + 63) / 64));
-    return f.scale0 != nullptr ? finish_w8<DT, MODE, true>(f, grid, stream) : finish_w8<DT, MODE, false>(f, grid, stream);
+    if constexpr (DT != kF32) {
+        if (f.scale0 != nullptr) return finish_w8<DT, MODE, true>(f, grid, stream);
+    }
+    return finish_w8<DT, MODE, false>(f, grid, stream);
 }
 template <int DT>
 hipError_t finish_dt(int mode, const DecFinish& f, hipStream_t stream) {
@@ -771,6 +906,7 @@ hipError_t launch_dec_finish(int mode, int dtype, const DecFinish& f, hipStream_
         return hipErrorInvalidValue;
     if (dtype == kBF16) return finish_dt<kBF16>(mode, f, stream);
     if (dtype == kF16) return finish_dt<kF16>(mode, f, stream);
+    if (dtype == kF32) return finish_dt<kF32>(mode, f, stream);
     return hipErrorInvalidValue;
 }
 

@@ -173,7 +173,7 @@ int candle_moe_set_combine_policy(int policy);
  *     128x128 tile would give the down GEMM fewer tiles than CUs, as with
  *     Nomic's hidden_dim 768),
  * 14 = 128x256 (BK 32, two workgroups per CU);
- * 18 = the decode kernels (f16 / bf16 / fp8, at most 1024 pairs and 4096
+ * 18 = the decode kernels (f16 / bf16 / f32 / fp8, at most 1024 pairs and 4096
  *     experts): no grouping launch (each workgroup groups the pairs in LDS),
  *     weights loaded straight into registers (transposed there for the API
  *     layout), K split across the waves of a workgroup and, for large
@@ -182,8 +182,10 @@ int candle_moe_set_combine_policy(int policy);
  * <= 128 rows per expert where the 256x256 tile would give few workgroups,
  * 14 for < 1024 rows per expert with hidden_dim <= 2048 when the down GEMM
  * has at least two 128x256 tiles per CU, else 7.
- * f32 (vector FMA): 15 = 32x128 tile, 16 = 128x128 tile, both with K splits
- * when the tiles are few; by default 15 for <= 32 rows per expert, else 16
+ * f32 (products on the bf16 matrix cores, each value split into three bf16
+ * parts): 15 = 32x128 tile, 16 = 128x128 tile, both with K splits when the
+ * tiles are few, and 18; by default 18 as for 16-bit weights (hidden_dim and
+ * intermediate_dim multiples of 8), 15 for <= 64 rows per expert, else 16
  * (the scalar 64x64 kernel 0 when hidden_dim or intermediate_dim is not a
  * multiple of 4 or an operand is not 16-byte aligned).
  * 17 concerns fp8 weights only (candle_moe_fused_moe_fp8; fused_moe

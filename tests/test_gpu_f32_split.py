@@ -1,0 +1,82 @@
+"""f32 MoE on the bf16 matrix cores (three-part split): accuracy at tile and
+K-step edges, and inputs the split cannot hold.
+
+Error bound of the accuracy cases (2-norm, relative to the 64-bit result).
+Every product keeps all but 2^-26 of itself; the large part products are
+accumulated in f32, one rounding per 16 k: at K <= 512 per GEMM at most 32
+roundings of 2^-24 each in a worst case that random signs do not reach, twice
+(two GEMMs), plus a few ulp of the activation and the final roundings:
+2 * 32 * 2^-24 + 4 * 2^-23 = 4.3e-6. A dropped part product of relative size
+2^-16 or a bf16-rounded operand would show at 1e-5 and above.
+"""
+import numpy as np
+import pytest
+
+import candle_moe
+import oracle as O
+from helpers import moe_inputs, to_dev, from_dev
+
+pytestmark = pytest.mark.gpu
+
+REL = 4.3e-6
+
+
+def _forward(x, G, U, D, rw, ri, E, k, act, mt, tile):
+    import torch
+
+    try:
+        candle_moe.set_tile_policy(tile)
+        moe = candle_moe.FusedMoE.new(E, k, candle_moe.Activation(act))
+        out = moe.forward(to_dev(x), to_dev(G), to_dev(U), to_dev(D) if D is not None else None, to_dev(rw),
+                          to_dev(ri), mt)
+        torch.cuda.synchronize()
+        return from_dev(out)
+    finally:
+        candle_moe.set_tile_policy(0)
+
+
+# tile 0: the default (decode kernels up to 256 pairs), 15 / 16: 32- and
+# 128-row tiles; row counts around 16, 32, 64 and 128 per expert, columns
+# around 64 and 128, K around the 32- and 64-deep steps, single-expert runs
+@pytest.mark.parametrize("tile,T,H,I,E,k,mt", [
+    (0, 1, 8, 8, 1, 1, 0), (0, 1, 768, 96, 8, 2, 1), (0, 16, 104, 200, 1, 1, 0), (0, 17, 512, 136, 3, 2, 1),
+    (0, 33, 72, 264, 2, 2, 0), (0, 128, 128, 64, 8, 2, 1), (18, 70, 256, 72, 2, 1, 0), (18, 70, 264, 56, 2, 1, 1),
+    (15, 31, 60, 132, 1, 1, 0), (15, 65, 68, 124, 2, 1, 1), (15, 32, 512, 64, 1, 1, 0), (15, 9, 4, 4, 2, 2, 1),
+    (16, 127, 100, 68, 1, 1, 0), (16, 129, 132, 260, 1, 1, 1), (16, 65, 36, 128, 1, 1, 0), (16, 3, 512, 192, 2, 1, 1),
+])
+def test_f32_split_accuracy(tile, T, H, I, E, k, mt):
+    act = O.SILU if mt == 0 else O.GELU
+    x, G, U, D, rw, ri = moe_inputs(T, H, I, E, k, O.F32, 900 + T + H, mt)
+    got = _forward(x, G, U, D, rw, ri, E, k, act, mt, tile).astype(np.float64)
+    want = O.fused_moe(x, G, U, D, rw, ri, E=E, k=k, act=act, moe_type=mt, dtype=O.F32, mode=O.MODE_EXACT)
+    err = np.linalg.norm(got - want) / np.linalg.norm(want)
+    assert err <= REL, err
+
+
+@pytest.mark.parametrize("tile", [0, 15, 16])
+@pytest.mark.parametrize("mt", [O.QWEN3, O.NOMIC])
+def test_f32_split_non_finite_and_extreme_inputs(tile, mt):
+    # an infinity, a NaN, a value whose bf16 part would round to infinity and
+    # values whose low parts are subnormal: what f32 FMAs give. (ReLU: an
+    # infinite pre-activation stays infinite or becomes zero.)
+    T, H, I, E, k = 40, 64, 72, 2, 1
+    x, G, U, D, rw, ri = moe_inputs(T, H, I, E, k, O.F32, 950, mt)
+    x[3, 5] = np.inf
+    x[4, 7] = -np.inf
+    x[9, 0] = np.nan
+    x[10, 1] = np.float32(3.4e38)
+    x[11, :] *= np.float32(1e-34)
+    x[12, :] = 0.0
+    G[0, 6, 3] = np.float32(0.5)  # parts m and l are zero: inf * 0 must not appear
+    got = _forward(x, G, U, D, rw, ri, E, k, O.RELU, mt, tile)
+    want = O.fused_moe(x, G, U, D, rw, ri, E=E, k=k, act=O.RELU, moe_type=mt, dtype=O.F32, mode=O.MODE_F32ACC)
+    for t in range(T):
+        g, w = got[t].astype(np.float64), np.asarray(want[t], dtype=np.float64)
+        if t in (3, 4, 9):
+            assert np.array_equal(np.isnan(g), np.isnan(w)), t
+            fin = ~np.isnan(w)
+            assert np.array_equal(g[fin], w[fin]) or np.allclose(g[fin], w[fin], rtol=1e-4), t
+        else:
+            assert np.isfinite(w).all() == np.isfinite(g).all(), t
+            if np.isfinite(w).all():
+                assert np.linalg.norm(g - w) <= 1e-5 * np.linalg.norm(w) + 1e-44, t
