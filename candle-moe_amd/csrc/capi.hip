@@ -134,6 +134,7 @@ struct Problem {
     bool packed;  // pre-packed K-contiguous 16-bit weights (candle_moe_fused_moe_packed)
     int cfg;  // TileCfg of both GEMMs
     int BM;
+    int ext;  // rows past BM that a group's last row tile also takes (row_tiles)
     long long P;
     bool set_path;  // expert-set down projection (no atomics, no f32 accumulator)
     int nkeys;      // (E+1)^k expert-set keys
@@ -537,6 +538,9 @@ static int check_problem(int T, int H, int I, int E, int k, int act, uint32_t mo
     p.rows_path = p.cfg == kDecGemv ||
                   (!p.set_path && p.lds_family && p.dtype != kF32 && p.cfg != kLdsRows32 && p.cfg != kW8Gemv &&
                    (double)P * H * 2.0 <= kRowsMaxBytes);
+    // extended row tiles on the 16-bit LDS-DMA kernels that have them (not with
+    // the f32-atomic combine, whose kernels share the tile table)
+    p.ext = (p.set_path || p.rows_path) && !fp8 ? ext_rows_of(p.cfg) : 0;
     p.n_tiles1 = cdiv(I, gemm_tile_cols(p.moe_type == kQwen3 ? kGateUp : kFc1, p.cfg));
     // Decode fc1 (Nomic) likewise on 128-column tiles where the 256-column
     // ones would split K: T=16 / 64 16.8 -> 13.4, 15.2 -> 12.9 us. (The
@@ -822,9 +826,9 @@ static int run_moe(const Problem& p, const void* x, const void* gate, const void
     if (p.cfg == kDecGemv) return run_moe_dec(p, x, gate, up, down, rw, idx, out, overwrite, ws, L, s, f8);
     {
         // pairs by expert and, on the expert-set path, tokens by expert set
-        const GroupJob pj = pair_grouping_job(idx, p.P, p.E, p.BM, gb);
+        const GroupJob pj = pair_grouping_job(idx, p.P, p.E, p.BM, p.ext, gb);
         GroupJob tj = {};
-        if (p.set_path) tj = set_grouping_job(idx, p.T, p.k, p.E, p.nkeys, p.BM, tb, pair_dest);
+        if (p.set_path) tj = set_grouping_job(idx, p.T, p.k, p.E, p.nkeys, p.BM, p.ext, tb, pair_dest);
         ProfScope ps(kSlotGroup, s);
         const bool one = sync_zero && g_grouping_mode != 1 &&
                          (g_grouping_mode == 2 || grouping_blocks(p.P) <= kGroupOneMaxBlocks);
@@ -873,6 +877,7 @@ static int run_moe(const Problem& p, const void* x, const void* gate, const void
     g1.pair_dest = pair_dest;
     g1.fold_w = p.set_path ? 1 : 0;
     g1.n_experts = p.E;
+    g1.ext = p.ext;
     g1.seg_len = p.I;
     if (f8) {  // codes [E][I][H]: n-rows of H bytes
         g1.ldb = p.H;
@@ -1346,7 +1351,7 @@ int candle_moe_group_pairs(const void* expert_indices, int num_pairs, int num_ex
     ws += cm::a256_bytes((size_t)(mt > 0 ? mt : 1) * 4);
     gb.num_tiles = reinterpret_cast<int32_t*>(ws);
     const cm::GroupJob pj =
-        cm::pair_grouping_job(reinterpret_cast<const uint32_t*>(expert_indices), P, E, 256, gb);
+        cm::pair_grouping_job(reinterpret_cast<const uint32_t*>(expert_indices), P, E, 256, 0, gb);
     const hipError_t e = cm::launch_groupings(pj, nullptr, reinterpret_cast<hipStream_t>(stream));
     return e == hipSuccess ? CANDLE_MOE_OK : cm::hip_fail(e, "group_pairs launch");
 }

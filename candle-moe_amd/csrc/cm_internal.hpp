@@ -56,14 +56,14 @@ constexpr int kSetMaxKeys = 1024;
 struct GroupJob {
     const uint32_t* idx;
     long long items;
-    int k, E, nbins, ebits, BM, nb;
+    int k, E, nbins, ebits, BM, ext, nb;  // BM, ext: row tile height and extension (row_tiles)
     int small;
     GroupingBufs b;
     int32_t* pair_dest;
 };
-GroupJob pair_grouping_job(const uint32_t* idx, long long P, int E, int BM, const GroupingBufs& b);
-GroupJob set_grouping_job(const uint32_t* idx, int T, int k, int E, int nkeys, int BM, const GroupingBufs& b,
-                          int32_t* pair_dest);
+GroupJob pair_grouping_job(const uint32_t* idx, long long P, int E, int BM, int ext, const GroupingBufs& b);
+GroupJob set_grouping_job(const uint32_t* idx, int T, int k, int E, int nkeys, int BM, int ext,
+                          const GroupingBufs& b, int32_t* pair_dest);
 size_t a256_bytes(size_t x);  // x rounded up to 256 bytes
 // The pair grouping and optionally the token grouping: one launch when both
 // have at most kGroupSmallMax items, or when sync (4 ints, zero before the
@@ -136,9 +136,19 @@ struct GemmArgs {
     // 16-bit weights pre-packed K-contiguous ([N,K] per expert, ldb = K) for
     // every GEMM (candle_moe_fused_moe_packed); LDS-DMA kernels only
     int packed;
+    // rows past the tile height that a group's last row tile may also hold (the
+    // tile table was built with it): 0 or kTileExt
+    int ext;
 };
 constexpr int kTailMaxSplit = 8;
 constexpr int kTailMinKTiles = 8;  // K tiles per tail split at least (shorter splits lose to the fixup)
+// A launch of at most half a round (all its tiles in the tail): the splits'
+// partials (256 KB each, written through and read back with every CU doing so
+// at once) cost about 25 us, 1.5 us per K tile. Qwen3 down (24 K tiles)
+// T=700 / 1000 split in two 54.6 / 58.2, whole 43.6 / 47.4 us; behind full
+// rounds, where other CUs are still computing, the split pays (T=2048 / 4096
+// 73 / 120.5 against 79.2 / 126 us).
+constexpr int kTailAloneMinKTiles = 40;
 
 // Kernel shapes (the codes of candle_moe_set_tile_policy; the missing codes
 // belonged to measured variants that are not shipped and are rejected).
@@ -178,6 +188,14 @@ inline int tile_rows(int cfg) {
     if (cfg == kTileSimt) return 64;
     if (cfg == kLds256w8) return 256;
     return 128;  // kTile128, kLds128, kLds128x256o2, kF32Tile128
+}
+// Extended row tiles (moe_lds_gemm): a group's last tile also takes up to
+// kTileExt rows past its height. 0: the kernel has none.
+constexpr int kTileExt = 32;
+inline int ext_rows_of(int cfg) { return cfg == kLds128 || cfg == kLds128x256o2 ? kTileExt : 0; }
+// Row tiles of a group of n rows.
+__host__ __device__ inline int row_tiles(int n, int bm, int ext) {
+    return n <= 0 ? 0 : n <= bm ? 1 : (n - ext + bm - 1) / bm;
 }
 // kW8Gemv: 16-column blocks per wave; output columns of a workgroup whose 4
 // waves split K in kw parts; kw for a GEMM of K, N over `tiles` row tiles:

@@ -256,7 +256,8 @@ __device__ __forceinline__ bool splitk_fixup(const GemmArgs& a, f32x16 (&acc)[MB
 }
 
 // Work item of this workgroup under tail balance (GemmArgs::tail_cus = C > 0).
-// XCD x takes a contiguous range of nx of the `live` tiles, as xcd_logical;
+// (A launch that is all tail, full = 0, splits only from kTailAloneMinKTiles K
+// tiles on.) XCD x takes a contiguous range of nx of the `live` tiles, as xcd_logical;
 // its first nx - R (R = nx mod C) tiles run whole, in nx / C full rounds over
 // the XCD's C CUs. The R tiles of the last round are split along K into
 // S = min(C / R, 8, K tiles / 8) parts when R <= C / 2, so that R * S workgroups
@@ -272,7 +273,8 @@ __device__ __forceinline__ bool tail_item(int live, int C, int nk_all, int& tile
     const int base = xcd * per + (xcd < rem ? xcd : rem);
     const int R = nx % C, full = nx - R;
     int S = 1;
-    if (R > 0 && 2 * R <= C) S = min(min(C / R, kTailMaxSplit), nk_all / kTailMinKTiles);
+    if (R > 0 && 2 * R <= C && (full > 0 || nk_all >= kTailAloneMinKTiles))
+        S = min(min(C / R, kTailMaxSplit), nk_all / kTailMinKTiles);
     ks = 0;
     nsplit = 1;
     slot0 = ctr = 0;
@@ -468,11 +470,18 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& a, f32x16 (&acc)[M
 // SC (fp8 weights): the f32 sums are first scaled by the tile's column
 // scales sc0 (gate/up: gate's, sc1 up's), indexed by the output column in
 // the tile.
-template <int DT, int MODE, int BM, int BN, int WM, int WN, int MB, int NB, int NW, bool SC = false>
+// EXT > 0 (extended tiles): m_valid may reach BM + EXT; the extension rows'
+// blocks are accx[NX] (column blocks wm * NX .. of the wave's, weights wx by
+// row) and dst_rows has BM + EXT entries. Where LDS_BYTES holds BM + EXT rows
+// they go out with the others, else in a second pass. Gate/up with NX = 1: the
+// wave rows hold gate (0) and up (1) of the same columns; up comes over in f32
+// through the LDS past the rows.
+template <int DT, int MODE, int BM, int BN, int WM, int WN, int MB, int NB, int NW, bool SC, int EXT, int LDS_BYTES,
+          int NX>
 __device__ __forceinline__ void staged_epilogue(const GemmArgs& a, f32x16 (&acc)[MB][NB], char* tile_lds,
                                                 const int32_t* dst_rows, int m_valid, int nt, int wm, int wn,
-                                                int lane, const float* pre_w, const float* sc0 = nullptr,
-                                                const float* sc1 = nullptr) {
+                                                int lane, const float* pre_w, const float* sc0, const float* sc1,
+                                                f32x16 (&accx)[NX], const float* wx) {
     constexpr bool DUAL = (MODE == kGateUp);
     constexpr bool GATHER = (MODE == kGateUp || MODE == kFc1);
     constexpr bool ROWS = (MODE == kDownRows || MODE == kFc2Rows);
@@ -548,19 +557,90 @@ __device__ __forceinline__ void staged_epilogue(const GemmArgs& a, f32x16 (&acc)
             }
         }
     }
-    __syncthreads();
-    // (2) whole rows out
+    // (2) whole rows out: tile rows first .. first + n - 1, from LDS row 0
     constexpr int RPI = 64 / CPR;  // rows per wave instruction
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int c = lane % CPR;
     const int col = nt * W + c * 8;
     uint16_t* C = reinterpret_cast<uint16_t*>(a.C);
-    if (col < N) {
-        for (int r = wave * RPI + lane / CPR; r < m_valid; r += NW * RPI) {
-            const u32x4 v = *reinterpret_cast<const u32x4*>(tile_lds + r * RB + ((c ^ (r % CPR)) << 4));
-            *reinterpret_cast<u32x4*>(C + (long long)dst_rows[r] * N + col) = v;
+    auto rows_out = [&](int first, int n) {
+        if (col < N) {
+            for (int r = wave * RPI + lane / CPR; r < n; r += NW * RPI) {
+                const u32x4 v = *reinterpret_cast<const u32x4*>(tile_lds + r * RB + ((c ^ (r % CPR)) << 4));
+                *reinterpret_cast<u32x4*>(C + (long long)dst_rows[first + r] * N + col) = v;
+            }
+        }
+    };
+    if constexpr (EXT > 0) {
+        if (m_valid > BM) {
+            constexpr bool SPLIT_PAIR = DUAL && NX == 1;
+            constexpr bool FITS = (BM + EXT) * RB + (SPLIT_PAIR ? NW / 2 * 4096 : 0) <= LDS_BYTES;
+            static_assert(!SPLIT_PAIR || FITS, "gate / up exchange");
+            f32x4* xch = reinterpret_cast<f32x4*>(tile_lds + (BM + EXT) * RB) + wn * 64 + lane;
+            constexpr int STEP = NW / 2 * 64;
+            if constexpr (SPLIT_PAIR) {
+                if (wm == 1) {
+#pragma unroll
+                    for (int g = 0; g < 4; ++g)
+                        xch[g * STEP] = f32x4{accx[0][4 * g], accx[0][4 * g + 1], accx[0][4 * g + 2], accx[0][4 * g + 3]};
+                }
+                __syncthreads();
+            }
+            if constexpr (!FITS) {
+                __syncthreads();
+                rows_out(0, BM);
+                __syncthreads();
+            }
+            const int ml = (FITS ? BM : 0) + lr;
+            if constexpr (GATHER) {
+                const float ws = wx[lr];
+                with_act(a.act, [&](auto act_c) {
+                    constexpr int ACT = decltype(act_c)::value;
+                    constexpr int PX = SPLIT_PAIR ? 1 : DUAL ? NX / 2 : NX;  // output blocks
+                    if (!SPLIT_PAIR || wm == 0) {
+#pragma unroll
+                        for (int q = 0; q < PX; ++q) {
+                            // output columns of the wave's pair (block) wm * PX + q
+                            const int lbase = DUAL ? (wn * WN) / 2 + (SPLIT_PAIR ? 0 : wm * PX + q) * 32
+                                                   : wn * WN + (wm * NX + q) * 32;
+#pragma unroll
+                            for (int g = 0; g < 4; ++g) {
+                                f32x4 u = {1.f, 1.f, 1.f, 1.f};
+                                if constexpr (SPLIT_PAIR) u = xch[g * STEP];
+                                float h[4];
+#pragma unroll
+                                for (int j = 0; j < 4; ++j) {
+                                    if constexpr (SPLIT_PAIR) {
+                                        h[j] = act_t<ACT>(accx[0][4 * g + j]) * u[j];
+                                    } else if constexpr (DUAL) {
+                                        h[j] = act_t<ACT>(accx[2 * q][4 * g + j]) * accx[(2 * q + 1) % NX][4 * g + j];
+                                    } else {
+                                        h[j] = act_t<ACT>(accx[q][4 * g + j]);
+                                    }
+                                    h[j] *= ws;
+                                }
+                                put(ml, lbase + 8 * g + nsub, h[0], h[1], h[2], h[3]);
+                            }
+                        }
+                    }
+                });
+            } else {
+                const float ws = ROWS ? wx[lr] : 1.0f;
+#pragma unroll
+                for (int q = 0; q < NX; ++q)
+#pragma unroll
+                    for (int g = 0; g < 4; ++g)
+                        put(ml, wn * WN + (wm * NX + q) * 32 + 8 * g + nsub, ws * accx[q][4 * g],
+                            ws * accx[q][4 * g + 1], ws * accx[q][4 * g + 2], ws * accx[q][4 * g + 3]);
+            }
+            __syncthreads();
+            if constexpr (FITS) rows_out(0, m_valid);
+            else rows_out(BM, m_valid - BM);
+            return;
         }
     }
+    __syncthreads();
+    rows_out(0, m_valid);
 }
 
 // Expert-set down / fc2 in accumulate mode (out = dtype(out + acc), one

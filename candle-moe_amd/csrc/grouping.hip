@@ -336,7 +336,7 @@ __device__ void scatter_body(const GroupJob& j, int blk, int32_t* s_mem, int src
         if (active && r == 0) mine[b] = before + __popcll(peers);
         lrank[s] = before + r;
     }
-    for (int e = threadIdx.x; e < nbins; e += kGroupThreads) s_tb[e] = (s_tot[e] + BM - 1) / BM;
+    for (int e = threadIdx.x; e < nbins; e += kGroupThreads) s_tb[e] = row_tiles(s_tot[e], BM, j.ext);
     __syncthreads();
     int32_t total, tiles, largest;
     block_exclusive_scan2(s_tot, s_tb, nbins, s_part, total, tiles, largest);  // s_tot -> offsets
@@ -348,7 +348,7 @@ __device__ void scatter_body(const GroupJob& j, int blk, int32_t* s_mem, int src
         for (int e = threadIdx.x; e < nbins; e += kGroupThreads) {
             offsets[e] = s_tot[e];
             const int32_t c = (e + 1 < nbins ? s_tot[e + 1] : total) - s_tot[e];
-            const int32_t nt = (c + BM - 1) / BM;
+            const int32_t nt = row_tiles(c, BM, j.ext);
             for (int i = 0; i < nt; ++i) {
                 tile_row[s_tb[e] + i] = s_tot[e] + i * BM;
                 tile_exp[s_tb[e] + i] = e;
@@ -448,7 +448,7 @@ __device__ void small_body(const GroupJob& j, int32_t* s_mem) {
         int32_t c = 0;
         for (int w = 0; w < NW; ++w) c += s_cnt[w * nbins + e];
         s_off[e] = c;
-        s_tb[e] = (c + BM - 1) / BM;
+        s_tb[e] = row_tiles(c, BM, j.ext);
     }
     __syncthreads();
     int32_t total, tiles, largest;
@@ -456,7 +456,7 @@ __device__ void small_body(const GroupJob& j, int32_t* s_mem) {
     for (int e = threadIdx.x; e < nbins; e += kGroupThreads) {
         offsets[e] = s_off[e];
         const int32_t c = (e + 1 < nbins ? s_off[e + 1] : total) - s_off[e];
-        const int32_t nt = (c + BM - 1) / BM;
+        const int32_t nt = row_tiles(c, BM, j.ext);
         for (int i = 0; i < nt; ++i) {
             tile_row[s_tb[e] + i] = s_off[e] + i * BM;
             tile_exp[s_tb[e] + i] = e;
@@ -574,7 +574,7 @@ __global__ __launch_bounds__(kGroupThreads) void grouping_final_k(GroupJob A, Gr
     }
 }
 
-static GroupJob make_job(const uint32_t* idx, long long items, int k, int E, int nbins, int BM,
+static GroupJob make_job(const uint32_t* idx, long long items, int k, int E, int nbins, int BM, int ext,
                          const GroupingBufs& b, int32_t* pair_dest) {
     GroupJob j = {};
     j.idx = idx;
@@ -583,6 +583,7 @@ static GroupJob make_job(const uint32_t* idx, long long items, int k, int E, int
     j.E = E;
     j.nbins = nbins;
     j.BM = BM;
+    j.ext = ext;
     j.b = b;
     j.pair_dest = pair_dest;
     while ((1 << j.ebits) < nbins) ++j.ebits;
@@ -593,13 +594,13 @@ static GroupJob make_job(const uint32_t* idx, long long items, int k, int E, int
     return j;
 }
 
-GroupJob pair_grouping_job(const uint32_t* idx, long long P, int E, int BM, const GroupingBufs& b) {
-    return make_job(idx, P, 1, E, E, BM, b, nullptr);
+GroupJob pair_grouping_job(const uint32_t* idx, long long P, int E, int BM, int ext, const GroupingBufs& b) {
+    return make_job(idx, P, 1, E, E, BM, ext, b, nullptr);
 }
 
-GroupJob set_grouping_job(const uint32_t* idx, int T, int k, int E, int nkeys, int BM, const GroupingBufs& b,
-                          int32_t* pair_dest) {
-    return make_job(idx, T, k, E, nkeys, BM, b, pair_dest);
+GroupJob set_grouping_job(const uint32_t* idx, int T, int k, int E, int nkeys, int BM, int ext,
+                          const GroupingBufs& b, int32_t* pair_dest) {
+    return make_job(idx, T, k, E, nkeys, BM, ext, b, pair_dest);
 }
 
 template <int KB>

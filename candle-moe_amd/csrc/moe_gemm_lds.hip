@@ -29,8 +29,24 @@ namespace cm {
 
 using namespace lds;
 
+// Extended tiles (EXT = 32; a.ext says whether the tile table uses them): the
+// last row tile of a group also takes the up to 32 rows past BM, instead of
+// leaving them to a tile of their own, which would stream the whole weight
+// panel again for a few rows: a tile's time is mostly that stream (with 64 of
+// 256 rows 0.75 of the full tile's), and routing puts many groups just past a
+// multiple of BM (T*k/E rows each, give or take a standard deviation).
+// The 32 rows are one more 32-row block against all BN columns, shared out
+// over the waves: wave (wm, wn) multiplies it with NB / 2 of the NB column
+// blocks it reads anyway (those from index wm * NB / 2), one more A fragment
+// and NB / 2 more MFMAs per k16 step. The K loop exists twice, with and without
+// the block, chosen per tile; the block's rows are stored directly.
+// Measured (gate/up / down): Qwen3 T=500 on 128x128 tiles 97 / 46 -> 66 / 32
+// us, Qwen3-30B-A3B T=2000 / 4096 on 128x256 tiles 212 / 110 -> 184 / 98 and 298
+// / 165 -> 283 / 158 us. Not on the 256x256 kernel: its extended tiles took 13 %
+// longer, which the fewer tiles repaid only here and there (Qwen3 T=4096 203 /
+// 136 -> 213 / 122, Nomic T=8191 112 / 80 -> 115 / 79 us).
 template <int DT, int BM, int BN, int BK, int NST, int NW, int MODE, int WGM = 2, int OCC = 1, bool W8 = false,
-          bool PK = false>
+          bool PK = false, int EXT = 0>
 __global__ __launch_bounds__(64 * NW, OCC) void moe_lds_gemm(GemmArgs a) {
     // NW waves in WGM rows: 4 in a 2x2 layout (one per SIMD), 8 in 2x4 (two
     // per SIMD, so one wave's MFMAs cover the other's LDS, DMA and VALU work),
@@ -64,7 +80,13 @@ __global__ __launch_bounds__(64 * NW, OCC) void moe_lds_gemm(GemmArgs a) {
     constexpr int KCH = KROW / 16;
     constexpr int KRPI = 1024 / KROW;  // fp8 n-rows per DMA instruction
     constexpr int B_BYTES = W8 ? BN * KROW : BN * AROW;
-    constexpr int STAGE = A_BYTES + B_BYTES;
+    static_assert(EXT == 0 || (EXT == 32 && NW == 4 && BM == 128 && WGM == 2 && NB % 2 == 0 && !ATOMIC && !W8),
+                  "extended tiles");
+    constexpr bool EX = EXT > 0;
+    constexpr int NX = EX ? NB / 2 : 1;     // column blocks of the extension rows per wave
+    constexpr int X_INS = EX ? EXT / RPA : 1;  // DMA instructions of the extension rows (per stage)
+    constexpr int X_OFF = A_BYTES + B_BYTES;
+    constexpr int STAGE = A_BYTES + B_BYTES + EXT * AROW;
     constexpr int A_INS = A_BYTES / (1024 * NW);  // DMA instructions per wave per stage
     constexpr int B_INS = B_BYTES / (1024 * NW);
     constexpr int LOADS = A_INS + B_INS;
@@ -92,7 +114,7 @@ __global__ __launch_bounds__(64 * NW, OCC) void moe_lds_gemm(GemmArgs a) {
                   "fp8 B tile");
     static_assert(LOADS * (NST - 2) < 64, "vmcnt range");
     __shared__ __attribute__((aligned(1024))) char smem[NST * STAGE];
-    __shared__ int32_t s_tok[(ATOMIC || SET) ? BM : 1];
+    __shared__ int32_t s_tok[(ATOMIC || SET) ? BM + EXT : 1];
     __shared__ float s_w[ATOMIC ? BM : 1];
     __shared__ float s_sc[W8 ? BN : 1];
     // fp8 expert sets: unit u_j[col] of segment j's column (its expert's
@@ -102,7 +124,8 @@ __global__ __launch_bounds__(64 * NW, OCC) void moe_lds_gemm(GemmArgs a) {
     // staged (row-contiguous) epilogue of the large tiles, see staged_epilogue
     constexpr bool STAGED = SWAP && BM >= 128;
     static_assert(!STAGED || NST * STAGE >= BM * (DUAL ? BN / 2 : BN) * 2, "output tile fits the stages");
-    __shared__ int32_t s_dst[STAGED ? BM : 1];
+    __shared__ int32_t s_dst[STAGED ? BM + EXT : 1];
+    __shared__ float s_wx[EX ? EXT : 1];  // routing weights of the extension rows
 
     // workgroup -> (output tile, K split); every workgroup first clears its
     // share of zero_f32 (the accumulator of the GEMM that follows)
@@ -126,7 +149,10 @@ __global__ __launch_bounds__(64 * NW, OCC) void moe_lds_gemm(GemmArgs a) {
     const int mt = tile / a.n_tiles, nt = tile - mt * a.n_tiles;
     const int r0 = a.tile_row[mt];
     const int grp = a.tile_exp[mt];
-    const int m_valid = min(BM, a.offsets[grp + 1] - r0);
+    // (extended tables: the group's last tile holds up to BM + EXT rows)
+    const int m_left = a.offsets[grp + 1] - r0;
+    const int m_valid = EX && m_left <= BM + a.ext ? m_left : min(BM, m_left);
+    const bool ext_rows = EX && m_valid > BM;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave / WGN, wn = wave % WGN;
@@ -170,6 +196,22 @@ __global__ __launch_bounds__(64 * NW, OCC) void moe_lds_gemm(GemmArgs a) {
             a_off[i] = r < m_valid ? ((uint32_t)(r0 + r) * (uint32_t)a_pitch + (uint32_t)kc) * 2u : kOob;
         }
     }
+    // extension rows: instruction wave % X_INS of X_INS (every wave issues
+    // one, so that the waves' DMA counts stay equal; repeats write the same
+    // bytes)
+    const int x_q = EX ? wave % X_INS : 0;
+    uint32_t x_off = kOob;
+    auto set_x_off = [&]() {
+        const int xr = RPA * x_q + lane / ACH;  // row of the block
+        const int r = BM + xr;
+        const int kc = a_swz<ACH>(xr, lane % ACH) * 8;
+        if constexpr (GATHER) {
+            const int src = a.sorted_pair[min(r0 + r, a.sorted_n - 1)] / a.k_top;
+            x_off = ((uint32_t)src * (uint32_t)a_pitch + (uint32_t)kc) * 2u;
+        } else {
+            x_off = r < m_valid ? ((uint32_t)(r0 + r) * (uint32_t)a_pitch + (uint32_t)kc) * 2u : kOob;
+        }
+    };
     // B [N,K]: like A over the column tile's rows n. B [K,N]: instruction i
     // (i % SUB_INS within sub-tile i / SUB_INS) covers k-rows RPI*q ..
     // RPI*q+RPI-1 of the tile, q = NW*(i % SUB_INS) + wave.
@@ -225,8 +267,8 @@ __global__ __launch_bounds__(64 * NW, OCC) void moe_lds_gemm(GemmArgs a) {
     weights_rsrc(seg_exp[0], rB0, rB1);
 
     // DMA instructions lo .. hi-1 of this wave's LOADS for the tile at k0
-    // (A instructions first, then B).
-    auto issue_range = [&](int stage, int k0, int lo, int hi) {
+    // (A instructions first, then B), then the extension rows' (xrows).
+    auto issue_range = [&](int stage, int k0, int lo, int hi, bool xrows) {
         const uint32_t sA = smem_base + stage * STAGE;
         const uint32_t sB = sA + A_BYTES;
         int kk = k0, klim = K;
@@ -265,7 +307,16 @@ __global__ __launch_bounds__(64 * NW, OCC) void moe_lds_gemm(GemmArgs a) {
                     dma16s(sub ? rB1 : rB0, sB + sub * SUB_BYTES + (NW * (i % SUB_INS) + wave) * 1024, b_off[i], sb);
                 }
             }
+            if constexpr (EX) {
+                if (xrows) dma16s(rA, sA + X_OFF + x_q * 1024, x_off, sa);
+            }
         } else {
+            if constexpr (EX) {
+                if (xrows) {
+                    const bool in = k0 + a_swz<ACH>(RPA * x_q + lane / ACH, lane % ACH) * 8 < K;
+                    dma16s(rA, sA + X_OFF + x_q * 1024, in ? x_off : kOob, sa);
+                }
+            }
             // K tail: every lane's chunk is checked against the operand's K
 #pragma unroll
             for (int i = 0; i < A_INS; ++i) {
@@ -299,7 +350,26 @@ __global__ __launch_bounds__(64 * NW, OCC) void moe_lds_gemm(GemmArgs a) {
             }
         }
     };
-    auto issue = [&](int stage, int k0) { issue_range(stage, k0, 0, LOADS); };
+    auto issue = [&](int stage, int k0, bool xrows) { issue_range(stage, k0, 0, LOADS, xrows); };
+    // output rows and weights of the extension rows, for the epilogue
+    auto stage_x_rows = [&]() {
+        if constexpr (GATHER || ROWS) {
+            if (wave == 0 && lane < EXT) {
+                const int r = r0 + (BM + lane < m_valid ? BM + lane : 0);
+                const int p = a.sorted_pair[r];
+                s_dst[BM + lane] = ROWS ? p : a.pair_dest ? a.pair_dest[p] : r;
+                s_wx[lane] = (ROWS || a.fold_w) ? a.routing_w[p] : 1.0f;
+            }
+        }
+    };
+    // the first K tile's DMA goes out before it is known whether the tile is
+    // extended (its group's end is still being loaded); the extension rows'
+    // share of it follows
+    auto issue_first_x = [&](int k0) {
+        set_x_off();
+        const bool in = k0 + BK <= K || k0 + a_swz<ACH>(RPA * x_q + lane / ACH, lane % ACH) * 8 < K;
+        dma16s(rA, smem_base + X_OFF + x_q * 1024, in ? x_off : kOob, (uint32_t)k0 * 2u);
+    };
 
     f32x16 acc[MB][NB];
 #pragma unroll
@@ -308,6 +378,11 @@ __global__ __launch_bounds__(64 * NW, OCC) void moe_lds_gemm(GemmArgs a) {
         for (int j = 0; j < NB; ++j)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+    f32x16 accx[NX];  // extension rows x this wave's column blocks
+#pragma unroll
+    for (int j = 0; j < NX; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) accx[j][r] = 0.0f;
 
     // fragment addresses (bytes inside a stage) that do not depend on kk
     const int lr = lane & 31, lh = lane >> 5;
@@ -360,6 +435,19 @@ __global__ __launch_bounds__(64 * NW, OCC) void moe_lds_gemm(GemmArgs a) {
                 else acc[mb][nb] = mfma32<DT>(af[mb], bfr[nb], acc[mb][nb]);
             }
     };
+    // the extension rows' A fragment of one k16 step, and its MFMAs
+    auto load_x = [&](const char* sA, int kk, u32x4& xf) {
+        xf = *reinterpret_cast<const u32x4*>(sA + X_OFF + lr * AROW + a_swz<ACH>(lr, kk * 2 + lh) * 16);
+    };
+    auto mfma_x = [&](const u32x4& xf, const u32x4 (&bfr)[NB]) {
+#pragma unroll
+        for (int j = 0; j < NX; ++j) {
+            u32x4 b;
+#pragma unroll
+            for (int d = 0; d < 4; ++d) b[d] = wm == 0 ? bfr[j][d] : bfr[(NX + j) % NB][d];
+            accx[j] = mfma32<DT>(b, xf, accx[j]);
+        }
+    };
     // fp8 expert sets: per-column unit changes of the accumulators. Lane l
     // holds, for block nb and register group g, columns wn*WN + nb*32 + 8g +
     // 4(l/32) .. +3 (the swapped MFMA layout), the same for every mb.
@@ -395,13 +483,16 @@ __global__ __launch_bounds__(64 * NW, OCC) void moe_lds_gemm(GemmArgs a) {
     constexpr int MFMA_PER_STEP = MB * NB;
     // Pin the schedule of one region: one MFMA, then one LDS read, while
     // reads remain, then the remaining MFMAs (masks: 0x8 MFMA, 0x100 DS read).
-    auto interleave = [&]() {
+    // (x: std::true_type with the extension rows' block)
+    auto interleave = [&](auto x) {
+        constexpr int XM = decltype(x)::value ? NX : 0, XD = decltype(x)::value ? 1 : 0;
 #pragma unroll
-        for (int i = 0; i < MFMA_PER_STEP; ++i) {
+        for (int i = 0; i < MFMA_PER_STEP + XM; ++i) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            if (i < DS_PER_STEP) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            if (i < DS_PER_STEP + XD) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
         }
     };
+    const std::false_type no_x{};
     // KSTEPS k16 steps per stage; the fragments of step kk+1 are read while
     // the MFMAs of step kk run (two register sets).
     // 8 waves: the waves of row group 1 issue the whole DMA of the next tile
@@ -411,7 +502,7 @@ __global__ __launch_bounds__(64 * NW, OCC) void moe_lds_gemm(GemmArgs a) {
     // DMA too little time before the next barrier).
     auto dma_slice = [&](int ds, int dk, int step) {
         if constexpr (NW == 8) {
-            if (step == 0 && ds >= 0) issue_range(ds, dk, 0, LOADS);
+            if (step == 0 && ds >= 0) issue_range(ds, dk, 0, LOADS, false);
             __builtin_amdgcn_sched_barrier(0);
         }
     };
@@ -497,19 +588,19 @@ __global__ __launch_bounds__(64 * NW, OCC) void moe_lds_gemm(GemmArgs a) {
         load_w8(sA, sB, 1, af1, br1);
         cvt(br0);
         mfma_step(af0, bfr);
-        interleave();
+        interleave(no_x);
         __builtin_amdgcn_sched_barrier(0);
         dma_slice(ds, dk, 0);
         load_w8(sA, sB, 2, af0, br0);
         cvt(br1);
         mfma_step(af1, bfr);
-        interleave();
+        interleave(no_x);
         __builtin_amdgcn_sched_barrier(0);
         dma_slice(ds, dk, 1);
         load_w8(sA, sB, 3, af1, br1);
         cvt(br0);
         mfma_step(af0, bfr);
-        interleave();
+        interleave(no_x);
         __builtin_amdgcn_sched_barrier(0);
         dma_slice(ds, dk, 2);
         cvt(br1);
@@ -517,7 +608,8 @@ __global__ __launch_bounds__(64 * NW, OCC) void moe_lds_gemm(GemmArgs a) {
         __builtin_amdgcn_sched_barrier(0);
         dma_slice(ds, dk, KSTEPS - 1);
     };
-    auto compute = [&](int stage, int ds, int dk) {
+    auto compute = [&](auto x, int stage, int ds, int dk) {
+        constexpr bool X = decltype(x)::value;
         if (!rows_live) {
 #pragma unroll
             for (int st = 0; st < KSTEPS; ++st) dma_slice(ds, dk, st);
@@ -525,27 +617,34 @@ __global__ __launch_bounds__(64 * NW, OCC) void moe_lds_gemm(GemmArgs a) {
         }
         const char* sA = smem + stage * STAGE;
         const char* sB = sA + A_BYTES;
-        u32x4 af0[MB], bf0[NB], af1[MB], bf1[NB];
+        u32x4 af0[MB], bf0[NB], af1[MB], bf1[NB], xf;
+        // (the extension rows' fragment is read at the start of its own step,
+        // whose other MFMAs cover it: no second register set)
+        auto mfmas = [&](const u32x4 (&af)[MB], const u32x4 (&bf)[NB], int kk) {
+            if constexpr (X) load_x(sA, kk, xf);
+            mfma_step(af, bf);
+            if constexpr (X) mfma_x(xf, bf);
+        };
         load_frags(sA, sB, 0, af0, bf0);
         __builtin_amdgcn_sched_barrier(0);
         load_frags(sA, sB, 1, af1, bf1);
-        mfma_step(af0, bf0);
-        interleave();
+        mfmas(af0, bf0, 0);
+        interleave(x);
         __builtin_amdgcn_sched_barrier(0);
         dma_slice(ds, dk, 0);
         if constexpr (KSTEPS == 4) {
             load_frags(sA, sB, 2, af0, bf0);
-            mfma_step(af1, bf1);
-            interleave();
+            mfmas(af1, bf1, 1);
+            interleave(x);
             __builtin_amdgcn_sched_barrier(0);
             dma_slice(ds, dk, 1);
             load_frags(sA, sB, 3, af1, bf1);
-            mfma_step(af0, bf0);
-            interleave();
+            mfmas(af0, bf0, 2);
+            interleave(x);
             __builtin_amdgcn_sched_barrier(0);
             dma_slice(ds, dk, 2);
         }
-        mfma_step(af1, bf1);
+        mfmas(af1, bf1, KSTEPS - 1);
         __builtin_amdgcn_sched_barrier(0);
         dma_slice(ds, dk, KSTEPS - 1);
     };
@@ -570,7 +669,7 @@ __global__ __launch_bounds__(64 * NW, OCC) void moe_lds_gemm(GemmArgs a) {
         }
     }
     if constexpr (SET) {
-        if (tid < BM) s_tok[tid] = a.tok_sorted[r0 + (tid < m_valid ? tid : 0)];
+        for (int r = tid; r < BM + EXT; r += 64 * NW) s_tok[r] = a.tok_sorted[r0 + (r < m_valid ? r : 0)];
     }
     // gate/up, fc1: the epilogue's output rows and routing weights (two
     // dependent reads per row), loaded now so that they are long done when the
@@ -593,7 +692,6 @@ __global__ __launch_bounds__(64 * NW, OCC) void moe_lds_gemm(GemmArgs a) {
             }
         }
     }
-
     // Stage hand-over, one barrier per K tile: wait for this wave's DMA of
     // stage kt (the NST-2 newer stages may stay in flight) and for its own
     // LDS reads of stage kt-1, then the barrier makes both block-wide; only
@@ -604,6 +702,7 @@ __global__ __launch_bounds__(64 * NW, OCC) void moe_lds_gemm(GemmArgs a) {
     const int kt0 = min(nk_all, ks * per_split);
     const int nk = min(nk_all, kt0 + per_split) - kt0;
 
+    if (nk > 0) issue(0, kt0 * BK, false);
     if constexpr (NW == 4 && !GATHER && !W8) {
         // 4-wave down / fc2 kernels: hand-over one k16 step early. The
         // barrier of tile kt+1 sits before the MFMAs of tile kt's last k16
@@ -619,73 +718,96 @@ __global__ __launch_bounds__(64 * NW, OCC) void moe_lds_gemm(GemmArgs a) {
         //   and its LDS reads of tile kt -> barrier -> DMA of tile kt+NST into
         //   tile kt's slot -> fragments of tile kt+1 step 0 under the MFMAs of
         //   tile kt's last step.
+        auto run = [&](auto x) {
+        constexpr bool X = decltype(x)::value;
         // wait for the DMA of the tile with `newer` of this wave's tiles
         // issued after it
-        auto wait_tile = [&](int newer) { wait_stage<LOADS, NST - 2>(newer); };
-        u32x4 af0[MB], bf0[NB], af1[MB], bf1[NB];
+        auto wait_tile = [&](int newer) { wait_stage<LOADS + (X ? 1 : 0), NST - 2>(newer); };
+        u32x4 af0[MB], bf0[NB], af1[MB], bf1[NB], xf;
+        auto mfmas = [&](const u32x4 (&af)[MB], const u32x4 (&bf)[NB], const char* sA, int kk) {
+            if constexpr (X) load_x(sA, kk, xf);
+            mfma_step(af, bf);
+            if constexpr (X) mfma_x(xf, bf);
+        };
+        if constexpr (X) {
+            if (nk > 0) issue_first_x(kt0 * BK);
+        }
 #pragma unroll
-        for (int s = 0; s < NST - 1; ++s)
-            if (s < nk) issue(s, (kt0 + s) * BK);
+        for (int s = 1; s < NST - 1; ++s)
+            if (s < nk) issue(s, (kt0 + s) * BK, X);
+        if constexpr (X) stage_x_rows();
         if (nk > 0) {
             wait_tile(min(NST - 2, nk - 1));
             wait_lgkm0();
             block_barrier();
-            if (NST - 1 < nk) issue(NST - 1, (kt0 + NST - 1) * BK);
+            if (NST - 1 < nk) issue(NST - 1, (kt0 + NST - 1) * BK, X);
             if (rows_live) load_frags(smem, smem + A_BYTES, 0, af0, bf0);
         }
         for (int kt = 0; kt < nk; ++kt) {
             const int st = kt % NST;
             const char* sA = smem + st * STAGE;
             const char* sB = sA + A_BYTES;
+            u32x4 xl;  // (the last step's, read before its stage is handed back)
             if (rows_live) {
                 load_frags(sA, sB, 1, af1, bf1);
-                mfma_step(af0, bf0);
-                interleave();
+                mfmas(af0, bf0, sA, 0);
+                interleave(x);
                 __builtin_amdgcn_sched_barrier(0);
                 if constexpr (KSTEPS == 4) {
                     load_frags(sA, sB, 2, af0, bf0);
-                    mfma_step(af1, bf1);
-                    interleave();
+                    mfmas(af1, bf1, sA, 1);
+                    interleave(x);
                     __builtin_amdgcn_sched_barrier(0);
                     load_frags(sA, sB, 3, af1, bf1);
-                    mfma_step(af0, bf0);
-                    interleave();
+                    mfmas(af0, bf0, sA, 2);
+                    interleave(x);
                     __builtin_amdgcn_sched_barrier(0);
                 }
+                if constexpr (X) load_x(sA, KSTEPS - 1, xl);
             }
             wait_tile(kt + 1 < nk ? min(NST - 2, nk - 2 - kt) : 0);
             wait_lgkm0();
             block_barrier();
             const int nx = kt + NST;
-            if (nx < nk) issue(st, (kt0 + nx) * BK);
+            if (nx < nk) issue(st, (kt0 + nx) * BK, X);
             if (rows_live) {
                 // (the last tile reads a stale stage: in bounds, unused)
                 const char* nA = smem + ((kt + 1) % NST) * STAGE;
                 load_frags(nA, nA + A_BYTES, 0, af0, bf0);
                 mfma_step(af1, bf1);
-                interleave();
+                if constexpr (X) mfma_x(xl, bf1);
+                interleave(x);
             }
             __builtin_amdgcn_sched_barrier(0);
         }
+        };
+        if (EX && ext_rows) run(std::integral_constant<bool, EX>{});
+        else run(no_x);
     } else {
     // fp8 expert sets: segment of the split's first K tile, and the K tile
     // at which the next one starts (segments are seg_kt whole K tiles)
     const int seg_kt = W8SET ? a.seg_len / BK : 1;
     int seg_cur = W8SET ? kt0 / seg_kt : 0;
     int seg_next = W8SET ? (seg_cur + 1) * seg_kt : 0;
+    auto run = [&](auto x) {
+    constexpr bool X = decltype(x)::value;
+    if constexpr (X) {
+        if (nk > 0) issue_first_x(kt0 * BK);
+    }
 #pragma unroll
-    for (int s = 0; s < NST - 1; ++s)
-        if (s < nk) issue(s, (kt0 + s) * BK);
+    for (int s = 1; s < NST - 1; ++s)
+        if (s < nk) issue(s, (kt0 + s) * BK, X);
+    if constexpr (X) stage_x_rows();
     for (int kt = 0; kt < nk; ++kt) {
         const int newer = min(NST - 2, nk - 1 - kt);  // stages issued after kt and before this wait
-        wait_stage<LOADS, NST - 2>(newer);
+        wait_stage<LOADS + (X ? 1 : 0), NST - 2>(newer);
         wait_lgkm0();
         block_barrier();
         const int ahead = kt + NST - 1;
         // row group 1 issues after its first k16 step (the decode kernels'
         // compute_w8 has no DMA slot)
         const bool late = NW == 8 && (!W8 || KSTEPS == 4) && wm == 1;
-        if (ahead < nk && !late) issue(ahead % NST, (kt0 + ahead) * BK);
+        if (ahead < nk && !late) issue(ahead % NST, (kt0 + ahead) * BK, X);
         if constexpr (W8SET) {
             // fp8 expert sets: the accumulators hold the current segment's
             // column units; entering segment j they are rescaled by
@@ -700,8 +822,11 @@ __global__ __launch_bounds__(64 * NW, OCC) void moe_lds_gemm(GemmArgs a) {
         if constexpr (W8 && NW == 8 && KSTEPS == 4)
             compute_w8i(kt % NST, (late && ahead < nk) ? ahead % NST : -1, (kt0 + ahead) * BK);
         else if constexpr (W8) compute_w8(kt % NST);
-        else compute(kt % NST, (late && ahead < nk) ? ahead % NST : -1, (kt0 + ahead) * BK);
+        else compute(x, kt % NST, (late && ahead < nk) ? ahead % NST : -1, (kt0 + ahead) * BK);
     }
+    };
+    if (EX && ext_rows) run(std::integral_constant<bool, EX>{});
+    else run(no_x);
     }
 
     if constexpr (W8SET) {
@@ -729,6 +854,18 @@ __global__ __launch_bounds__(64 * NW, OCC) void moe_lds_gemm(GemmArgs a) {
         sc0 = s_sc;
         if constexpr (DUAL) sc1 = s_sc + SUBN;
     }
+    // Accumulating expert-set GEMM: the extension rows, added directly (the
+    // other modes' go through the staged epilogue below).
+    if constexpr (EX && SET) {
+        if (ext_rows && !a.overwrite) {
+            f32x16 blk[1][NX];
+#pragma unroll
+            for (int j = 0; j < NX; ++j) blk[0][j] = accx[j];
+            tile_epilogue<DT, MODE, BN, 32, NX * 32, 1, NX>(a, blk, r0 + BM, m_valid - BM, nt, 0, 2 * wn + wm, lane,
+                                                            s_tok + BM, nullptr);
+        }
+    }
+    const int m_tile = EX ? min(m_valid, BM) : m_valid;  // the tile's own rows
     if constexpr (STAGED) {
         if (!SET || a.overwrite) {
             // output row of every tile row (gate/up, fc1: the pair's inter row;
@@ -740,18 +877,18 @@ __global__ __launch_bounds__(64 * NW, OCC) void moe_lds_gemm(GemmArgs a) {
                 }
             }
             __syncthreads();  // every wave is done with the stages
-            staged_epilogue<DT, MODE, BM, BN, WM, WN, MB, NB, NW, W8 && !SET>(a, acc, smem, SET ? s_tok : s_dst,
-                                                                             m_valid, nt, wm, wn, lane, pre_w, sc0,
-                                                                             sc1);
+            staged_epilogue<DT, MODE, BM, BN, WM, WN, MB, NB, NW, W8 && !SET, EXT, NST * STAGE, NX>(
+                a, acc, smem, SET ? s_tok : s_dst, EX ? m_valid : m_tile, nt, wm, wn, lane, pre_w, sc0, sc1, accx,
+                s_wx);
             return;
         }
         if constexpr (SET && BN == 256 && NST * STAGE >= BM * (BN / 2) * 4) {
             __syncthreads();  // every wave is done with the stages
-            staged_epilogue_acc<DT, BM, BN, WM, WN, MB, NB, NW>(a, acc, smem, s_tok, m_valid, nt, wm, wn, lane);
+            staged_epilogue_acc<DT, BM, BN, WM, WN, MB, NB, NW>(a, acc, smem, s_tok, m_tile, nt, wm, wn, lane);
             return;
         }
     }
-    tile_epilogue<DT, MODE, BN, WM, WN, MB, NB>(a, acc, r0, m_valid, nt, wm, wn, lane, s_tok, s_w,
+    tile_epilogue<DT, MODE, BN, WM, WN, MB, NB>(a, acc, r0, m_tile, nt, wm, wn, lane, s_tok, s_w,
                                                 (GATHER || ROWS) ? pre_dst : nullptr,
                                                 (GATHER || ROWS) ? pre_w : nullptr, sc0, sc1);
 }
@@ -766,12 +903,15 @@ hipError_t launch_lds_mode(int cfg, const GemmArgs& a, hipStream_t stream) {
     if (nwg_l > 0x7fffffffLL) return hipErrorInvalidValue;
     const int nwg = (int)nwg_l;
     if (nwg <= 0) return hipSuccess;
+    // extended row tiles, except for the f32-atomic combine
+    constexpr int X = (MODE == kDown || MODE == kFc2) ? 0 : kTileExt;
+    if (a.ext != 0 && (X == 0 || ext_rows_of(cfg) != a.ext)) return hipErrorInvalidValue;
     if constexpr (DT == kF32) {
         return hipErrorInvalidValue;
     } else {
         switch (cfg) {
             case kLds128:
-                hipLaunchKernelGGL((moe_lds_gemm<DT, 128, 128, 64, 4, 4, MODE, 2, 1, false, PK>), dim3(nwg), dim3(256),
+                hipLaunchKernelGGL((moe_lds_gemm<DT, 128, 128, 64, 4, 4, MODE, 2, 1, false, PK, X>), dim3(nwg), dim3(256),
                                    0, stream, a);
                 break;
             case kLds256w8:
@@ -792,7 +932,7 @@ hipError_t launch_lds_mode(int cfg, const GemmArgs& a, hipStream_t stream) {
             // two workgroups per CU (72 KB of LDS, at most 256 VGPRs each): one
             // workgroup's barrier and DMA issue overlap the other's MFMAs
             case kLds128x256o2:
-                hipLaunchKernelGGL((moe_lds_gemm<DT, 128, 256, 32, 3, 4, MODE, 2, 2, false, PK>), dim3(nwg),
+                hipLaunchKernelGGL((moe_lds_gemm<DT, 128, 256, 32, 3, 4, MODE, 2, 2, false, PK, X>), dim3(nwg),
                                    dim3(256), 0, stream, a);
                 break;
             default:
@@ -808,6 +948,7 @@ hipError_t launch_lds_mode(int cfg, const GemmArgs& a, hipStream_t stream) {
 // the 16-bit one) for larger batches
 template <int DT, int MODE>
 static hipError_t launch_w8_mode(int cfg, const GemmArgs& a, hipStream_t stream) {
+    if (a.ext != 0) return hipErrorInvalidValue;
     const long long tiles = (long long)a.m_tiles_max * a.n_tiles;
     if (cfg == kLds256w8) {
         if constexpr (MODE == kGateUp || MODE == kFc1 || MODE == kDownRows || MODE == kDownSet) {
