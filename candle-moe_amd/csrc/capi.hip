@@ -235,7 +235,7 @@ static long long set_tiles_max(const Problem& p) {
 
 // f32 decode calls: room for the K slices' partials (5 slices of Nomic's fc2
 // and 2 of Qwen3's gate/up at 256 pairs), kept whatever the batch, so that a
-// larger batch never needs a smaller workspace (dec_f32_floor).
+// larger batch never needs a smaller workspace.
 constexpr double kDecPartBytesF32 = 6.0 * 1024 * 1024;
 
 static size_t a256(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -314,12 +314,6 @@ static bool dec_gemv_fits(const Problem& p) {
            (long long)(p.I + 1024) * p.H * es < lim;
 }
 
-// Workspace of the largest f32 decode call of this layer (dtype, H, I, E, k):
-// the f32 tile kernels that larger batches take need less in places, and a
-// workspace grown (or sized by the caller) for a batch has to do for every
-// smaller one, also under graph capture, where it cannot grow.
-static size_t dec_f32_floor(const Problem& p);
-
 // Most K slices of a decode GEMM over N columns and K (the kernels choose
 // the slices from the experts a batch touches, up to this): cold weights
 // stream at the rate of the access pattern and of the workgroups reading
@@ -347,6 +341,12 @@ static int dec_cap() { return 2 * 8 * std::max(cus_per_xcd(), 32); }
 // the decode kernels against 115 / 126 / 134 / 149 us; Qwen3 T=128 (256
 // pairs) 102 against 115 us.
 constexpr long long kDecDefaultPairs = 256;
+// 16-bit prefill batches: rows per touched expert up to which nearly every
+// expert's rows fit one extended 128-row tile (160 rows: two standard
+// deviations of uniform routing above), and from which a 256-row tile often
+// spills into a second one (256 less 1.5 deviations).
+constexpr long long kOneTileRows = 136;
+constexpr long long kTwoTileRows = 232;
 
 // aligned16: input and weights start on 16-byte boundaries (the MFMA and f32
 // tiled kernels read them with 16-byte loads; otherwise the scalar kernel
@@ -383,16 +383,16 @@ static int check_problem(int T, int H, int I, int E, int k, int act, uint32_t mo
     // over T = 1 .. 32768 of the Qwen3, Qwen3-30B and Nomic shapes):
     //  * at most 32 (decode): the GEMMs stream each touched expert's weights
     //    once; the 32-row tile keeps the padding and the MFMA work small;
-    //  * at most 128, where the 256x256 tile would leave fewer than 256
-    //    workgroups (few experts): the 128x128 tile, which doubles to
-    //    quadruples the workgroups;
-    //  * fewer than 1024 with a hidden size of at most 2048 (short K loops of
-    //    the gate/up GEMM): the 128x256 tile, two workgroups per CU, so that
-    //    one's prologue, barriers and epilogue overlap the other's MFMAs --
-    //    if the down GEMM's 128x256 tiles fill both slots of every CU; with
-    //    a small hidden size (Nomic, H = 768: 3 column tiles) they do not,
-    //    and the 256x256 tile, whose partly filled last round is split along
-    //    K, is faster (Nomic T=2048 / 4096 steps 192 / 219 -> 119 / 198 us);
+    //  * up to kOneTileRows: 128-row tiles (128x128, or 128x256 with two
+    //    workgroups per CU where those fill the device), whose extension lets
+    //    most experts fit one tile; with short gate/up K loops up to 256;
+    //  * kTwoTileRows to 1024 with a hidden size of at most 2048: the 128x256
+    //    tile, so that one workgroup's prologue, barriers and epilogue overlap
+    //    the other's MFMAs -- if the down GEMM's 128x256 tiles fill both slots
+    //    of every CU; with a small hidden size (Nomic, H = 768: 3 column tiles)
+    //    they do not, and the 256x256 tile, whose partly filled last round is
+    //    split along K, is faster (Nomic T=2048 / 4096 steps 192 / 219 -> 119 /
+    //    198 us);
     //  * otherwise the 256x256 tile with 8 waves.
     // Expected live row tiles of a tile height: one per touched expert at
     // least, the rows over the tile height at least.
@@ -451,19 +451,42 @@ static int check_problem(int T, int H, int I, int E, int k, int act, uint32_t mo
             (g_tile_policy == kDecGemv && dec_gemv_fits(p)))
             p.cfg = g_tile_policy;
     } else if (p.mfma && !policy) {
+        const long long dev_wgs = 8LL * std::max(cus_per_xcd(), 32);
         const long long wgs256 = est_tiles(256) * cdiv(I, gemm_tile_cols(p.moe_type == kQwen3 ? kGateUp : kFc1, kLds256w8));
         if (P <= 32 * touched) p.cfg = P <= kDecDefaultPairs && dec_gemv_fits(p) ? kDecGemv : kLdsRows32;
         // up to 128 rows per touched expert, where the 128x128 tile would
         // leave the down GEMM too few tiles for the CUs (a narrow hidden
         // dimension: Nomic's 768) and its K is long enough to split (I >=
         // 1024), the 32-row kernel with its K splits: Nomic T=192 / 256 / 512
-        // steps 64.0 / 66.7 / 88.5 us on the 128x128 tile against 49.8 /
+        // steps 64.0 / 66.7 / 69.9 us on the 128x128 tile against 49.8 /
         // 55.9 / 75.1 us. (Its f32 atomics make these sizes' results vary in
-        // the last bits from call to call, as on the decode sizes it takes.)
-        else if (P <= 128 * touched && I >= 1024 && est_tiles(128) * cdiv(H, 128) < 8LL * std::max(cus_per_xcd(), 32))
+        // the last bits from call to call, as on the decode sizes it takes;
+        // they also keep the pairs' rows in f32 until the sum. With more down
+        // tiles the 128x128 tile is the faster one, H 1024 I 2048 16 experts
+        // T=500 60 against 77 us, but rounds each pair's row to 16 bits.)
+        else if (P <= 128 * touched && I >= 1024 && est_tiles(128) * cdiv(H, 128) < dev_wgs)
             p.cfg = kLdsRows32;
-        else if (wgs256 < 256 && P <= 128 * touched) p.cfg = kLds128;
-        else if (H <= 2048 && P < 1024 * touched && (long long)cdiv(H, 256) * est_tiles(128) >= 512)
+        // up to kOneTileRows rows per touched expert nearly every expert is one
+        // extended 128-row tile: 128x128 tiles while the gate/up GEMM has at
+        // most 1.5 of them per CU, else 128x256 with two workgroups per CU
+        // (steps, 128x128 / 128x256 / 256x256: Qwen3 T=520 106 / 153 / 138 us,
+        // H 2048 I 1408 16 experts top 4 T=300 92 / 95 / 107; H 2880 I 1000 32
+        // experts top 4 T=500 154 / 144 / 188, Qwen3-30B-A3B T=600 290 / 255 /
+        // 294 us; Qwen3 T=640, 160 rows: 159 / 155 / 140 us)
+        else if (P <= kOneTileRows * touched)
+            p.cfg = 2 * touched * cdiv(I, gemm_tile_cols(p.moe_type == kQwen3 ? kGateUp : kFc1, kLds128)) <= 3 * dev_wgs
+                        ? kLds128 : kLds128x256o2;
+        // short gate/up K loops (H <= 1024) below 256 rows per expert, where
+        // 256x256 tiles number less than the CUs: 128x128 (Nomic T=700 / 1000
+        // 81 / 81 against 85 / 95 us, H 1024 I 2048 16 experts T=1500 82
+        // against 107 us)
+        else if (H <= 1024 && P < 256 * touched && wgs256 < dev_wgs)
+            p.cfg = kLds128;
+        // (kOneTileRows .. kTwoTileRows rows: one 256-row tile per expert
+        // against two of 128: Qwen3-30B-A3B T=2600 / 3000 400 / 420 against 372
+        // / 382 us on 256x256; T=4096, 256 rows: 486 against 505 us)
+        else if (H <= 2048 && P < 1024 * touched && P >= kTwoTileRows * touched &&
+                 (long long)cdiv(H, 256) * est_tiles(128) >= 2 * dev_wgs)
             p.cfg = kLds128x256o2;
     }
     // (a forced decode kernel on sizes it does not take: the 32-row kernel)
@@ -625,12 +648,25 @@ static int check_problem(int T, int H, int I, int E, int k, int act, uint32_t mo
     return CANDLE_MOE_OK;
 }
 
-static size_t dec_f32_floor(const Problem& p) {
-    if (!p.f32_dec || p.cfg == kDecGemv) return 0;
-    Problem q;
-    const int T = (int)std::min<long long>(p.T, std::max<long long>(std::min<long long>(kDecDefaultPairs, 32LL * p.E) / p.k, 1));
-    if (check_problem(T, p.H, p.I, p.E, p.k, p.act, (uint32_t)p.moe_type, (uint32_t)p.dtype, q)) return 0;
-    return q.cfg == kDecGemv ? make_layout(q).total : 0;
+// Most workspace a smaller batch of the same layer (dtype, sizes, combine
+// policy) needs: the kernels that take smaller batches keep more of it in
+// places (decode partials by slice, K-split partials). A workspace allocated,
+// or sized by the caller, for a batch has to do for the smaller ones too, also
+// under graph capture, where it cannot grow. Asked at the largest batch of
+// each kernel's range.
+static size_t smaller_batches_ws(const Problem& p, bool fp8) {
+    const long long P_at[] = {kDecDefaultPairs, 32LL * p.E, 64LL * p.E, 128LL * p.E, kOneTileRows * p.E, 256LL * p.E - 1};
+    size_t most = 0;
+    for (long long P : P_at) {
+        const long long T = P / p.k;
+        Problem q;
+        if (T < 1 || T >= p.T ||
+            check_problem((int)T, p.H, p.I, p.E, p.k, p.act, (uint32_t)p.moe_type, (uint32_t)p.dtype, q, true, true, fp8,
+                          p.packed))
+            continue;
+        most = std::max(most, make_layout(q).total);
+    }
+    return most;
 }
 
 // fp8 expert weights of candle_moe_fused_moe_fp8 (codes [E][N][K], scales [E][N])
@@ -1009,24 +1045,22 @@ static std::vector<OwnedWs> g_ws;
 // (err = hipErrorStreamCaptureUnsupported): hipMallocAsync there would add an
 // allocation node to the caller's graph, memory the graph owns and releases
 // when it is destroyed, while this table would keep handing it out.
-// reserve: bytes wanted beyond need for later calls, not insisted on in a
-// capture.
-static OwnedWs* owned_ws_locked(int dev, hipStream_t s, size_t need, hipError_t& err, size_t reserve = 0) {
+// reserve: bytes to allocate at least, asked for when the workspace grows.
+template <class F>
+static OwnedWs* owned_ws_locked(int dev, hipStream_t s, size_t need, hipError_t& err, F&& reserve) {
     err = hipSuccess;
     OwnedWs* w = nullptr;
     for (auto& e : g_ws)
         if (e.device == dev && e.stream == s) w = &e;
-    if (w && w->bytes >= std::max(need, reserve)) return w;
+    if (w && w->bytes >= need) return w;
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone) {
-        if (w && w->bytes >= need) return w;
         err = hipErrorStreamCaptureUnsupported;
         return nullptr;
     }
-    need = std::max(need, reserve);
     // grow by at least 1.5x and to whole MiB, so that a slowly growing T
     // does not reallocate on every call
-    size_t want = need + need / 2;
+    size_t want = std::max(need + need / 2, (size_t)reserve());
     want = (want + (1u << 20) - 1) & ~(size_t)((1u << 20) - 1);
     void* mem = nullptr;
     err = hipMallocAsync(&mem, want, s);
@@ -1104,7 +1138,9 @@ int fused_moe_impl(const void* x, const void* gate, const void* up, const void* 
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return hip_fail(e, "fused_moe: hipGetDevice");
     std::lock_guard<std::mutex> lk(g_ws_mu);
-    OwnedWs* w = owned_ws_locked(dev, s, L.total, e, dec_f32_floor(p));
+    // (asked for only where the workspace has to grow)
+    const auto reserve = [&]() { return aligned16 ? smaller_batches_ws(p, f8 != nullptr) : (size_t)0; };
+    OwnedWs* w = owned_ws_locked(dev, s, L.total, e, reserve);
     if (!w) return ws_fail("fused_moe", L.total, e);
     return run_moe(p, x, gate, up, down, reinterpret_cast<const float*>(rw), reinterpret_cast<const uint32_t*>(idx),
                    out, overwrite, reinterpret_cast<char*>(w->ptr), s, f8, true);
@@ -1188,7 +1224,7 @@ size_t fused_moe_ws_size(int T, int H, int I, int E, int k, uint32_t dtype) {
         for (int al = 0; al < 2; ++al) {
             Problem p;
             if (check_problem(T, H, I, E, k, 0, mt, dtype, p, al != 0)) return 0;
-            most = std::max(most, std::max(make_layout(p).total, dec_f32_floor(p)));
+            most = std::max(most, std::max(make_layout(p).total, al ? smaller_batches_ws(p, false) : (size_t)0));
         }
     return most;
 }
@@ -1393,7 +1429,7 @@ int candle_moe_router_topk(const void* hidden, const void* router_weight, void* 
         e = hipGetDevice(&dev);
         if (e != hipSuccess) return cm::hip_fail(e, "router_topk: hipGetDevice");
         std::lock_guard<std::mutex> lk(cm::g_ws_mu);
-        cm::OwnedWs* w = cm::owned_ws_locked(dev, s, need, e);
+        cm::OwnedWs* w = cm::owned_ws_locked(dev, s, need, e, [] { return (size_t)0; });
         if (!w) return cm::ws_fail("router_topk", need, e);
         e = cm::launch_router_topk(hidden, router_weight, (int)dtype, reinterpret_cast<float*>(topk_weight),
                                    reinterpret_cast<uint32_t*>(topk_indices),

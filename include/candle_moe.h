@@ -178,10 +178,13 @@ int candle_moe_set_combine_policy(int policy);
  *     weights loaded straight into registers (transposed there for the API
  *     layout), K split across the waves of a workgroup and, for large
  *     gate/up streams, across workgroups; default for <= 32 rows per expert
- *     on average and at most 256 pairs (fp8: 128). By default 5 is taken for
- * <= 128 rows per expert where the 256x256 tile would give few workgroups,
- * 14 for < 1024 rows per expert with hidden_dim <= 2048 when the down GEMM
- * has at least two 128x256 tiles per CU, else 7.
+ *     on average and at most 256 pairs (fp8: 128).
+ * By default, up to 136 rows per expert 5 (14 where 5 would give the gate/up
+ * GEMM more than 1.5 tiles per CU), 5 also below 256 rows with hidden_dim <=
+ * 1024 and few 256x256 tiles, 14 for 232 to 1024 rows per expert with
+ * hidden_dim <= 2048 when the down GEMM has at least two 128x256 tiles per CU,
+ * else 7. On 5 and 14 the last row tile of an expert (or expert set) may hold
+ * up to 32 rows more than its 128.
  * f32 (products on the bf16 matrix cores, each value split into three bf16
  * parts): 15 = 32x128 tile, 16 = 128x128 tile, both with K splits when the
  * tiles are few, and 18; by default 18 as for 16-bit weights (hidden_dim and

@@ -1,0 +1,44 @@
+"""The 16-bit dispatch by rows per touched expert: kernel codes on both sides of
+each line, and workspaces past a line that do for the batches before it."""
+import pytest
+
+import candle_moe as cm
+
+# (H, I, E, k, pairs per expert) -> kernel code (moe_type 0, bf16, 256 CUs)
+EDGES = [
+    (4096, 1536, 8, 2, 32, 18),        # decode kernels: 256 pairs
+    (4096, 1536, 8, 2, 33, 5),         # 128x128 up to 136 rows
+    (4096, 1536, 8, 2, 136, 5),
+    (4096, 1536, 8, 2, 137, 7),        # above: one 256-row tile per expert
+    (2048, 768, 128, 8, 32, 12),
+    (2048, 768, 128, 8, 33, 14),       # more than 1.5 128x128 tiles per CU
+    (2048, 768, 128, 8, 136, 14),
+    (2048, 768, 128, 8, 137, 7),
+    (2048, 768, 128, 8, 231, 7),
+    (2048, 768, 128, 8, 232, 14),      # a 256-row tile often spills over
+    (2048, 768, 128, 8, 1023, 14),
+    (2048, 768, 128, 8, 1024, 7),
+    (1024, 1024, 16, 2, 128, 12),      # few down tiles: f32 atomics kept
+    (1024, 1024, 16, 2, 129, 5),
+    (1024, 1024, 16, 2, 255, 5),       # short gate/up K loops, few 256x256 tiles
+    (1024, 1024, 16, 2, 256, 7),
+]
+
+
+@pytest.mark.parametrize("H,I,E,k,rows,code", EDGES)
+def test_kernel_at_the_lines(H, I, E, k, rows, code):
+    T = rows * E // k
+    assert T * k == rows * E
+    assert cm.fused_moe_kernel(T, H, I, E, k, cm.DT_BF16) == code
+
+
+@pytest.mark.parametrize("dt", [cm.DT_BF16, cm.DT_F16, cm.DT_F32])
+@pytest.mark.parametrize("H,I,E,k", [(4096, 1536, 8, 2), (2048, 768, 128, 8), (768, 3072, 8, 2), (1024, 2048, 16, 2),
+                                     (520, 264, 5, 3)])
+def test_workspace_past_a_line(H, I, E, k, dt):
+    """Past a line the workspace still holds the largest batch before it."""
+    size = cm.lib().candle_moe_fused_moe_workspace_size
+    lines = sorted({256 // k} | {r * E // k for r in (32, 64, 128, 136)} | {(256 * E - 1) // k})
+    for i, T in enumerate(lines):
+        for larger in [T + 1] + lines[i + 1:] + [2 * lines[-1]]:
+            assert size(larger, H, I, E, k, dt) >= size(T, H, I, E, k, dt) > 0, (T, larger)
