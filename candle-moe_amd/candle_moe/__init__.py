@@ -75,11 +75,31 @@ class CmFusedMoE(ctypes.Structure):
 
 
 _lib = None
+# candle_moe._fast bound to _lib (csrc/torch_bindings.cpp), or None before the
+# library is loaded and where the module is not built: the calls below then
+# describe their tensors here.
+_native = None
+
+
+def _bind_native(L: ctypes.CDLL):
+    try:
+        import torch
+        from . import _fast as f
+    except ImportError:
+        return None
+    raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if raw_stream is None or torch.__version__.split("+")[0] != f.torch_version:
+        return None
+    addr = lambda fn: ctypes.cast(fn, ctypes.c_void_p).value  # noqa: E731
+    f.bind(addr(L.candle_moe_apply_topk_softmax_inplace), addr(L.candle_moe_fused_moe_forward),
+           addr(L.candle_moe_router_topk), addr(L.candle_moe_fused_moe_fp8), addr(L.candle_moe_fused_moe_packed),
+           raw_stream)
+    return f
 
 
 def lib() -> ctypes.CDLL:
     """The loaded HIP library (raises if it has not been built)."""
-    global _lib
+    global _lib, _native
     if _lib is None:
         if not os.path.exists(LIB_PATH):
             raise RuntimeError(
@@ -156,6 +176,7 @@ def lib() -> ctypes.CDLL:
         L.candle_moe_fused_moe_forward.restype = i32
         L.candle_moe_validate_fused_moe.argtypes = [mp, tp, tp, tp, tp, tp, tp, u32, tp]
         L.candle_moe_validate_fused_moe.restype = i32
+        _native = _bind_native(L)
         _lib = L
     return _lib
 
@@ -252,6 +273,10 @@ def apply_topk_softmax_inplace(gating_output, topk_weight, topk_indices, token_e
     gating_output [T, E]; topk_weight [T, k] of the same dtype (f32, f16 or
     bf16); topk_indices / token_expert_indices [T, k] u32 (int32 accepted).
     """
+    if _native is not None:
+        rc = _native.topk(gating_output, topk_weight, topk_indices, token_expert_indices)
+        if rc is not None:
+            return check(rc)
     g, w, i, ei = (describe(t) for t in (gating_output, topk_weight, topk_indices, token_expert_indices))
     check(lib().candle_moe_apply_topk_softmax_inplace(
         ctypes.byref(g), ctypes.byref(w), ctypes.byref(i), ctypes.byref(ei), _stream_for(gating_output)))
@@ -289,6 +314,10 @@ def router_topk(hidden, router_weight, topk_weight, topk_indices, token_expert_i
     layout) of one dtype, contiguous; logits = dtype(hidden @ router_weight.T)
     with f32 accumulation; outputs as apply_topk_softmax_inplace with f32
     topk_weight [T, k]."""
+    if _native is not None:
+        rc = _native.router(hidden, router_weight, topk_weight, topk_indices, token_expert_indices)
+        if rc is not None:
+            return check(rc)
     for t in (hidden, router_weight, topk_weight, topk_indices, token_expert_indices):
         if not t.is_contiguous():
             raise CandleMoeError(CANDLE_MOE_ERR_INVALID, "router_topk: tensors must be contiguous")
@@ -354,6 +383,11 @@ def fused_moe_fp8(input, gate_q, up_q, down_q, gate_scale, up_scale, down_scale,
     contiguous and on input's device; the codes are uint8 and the scales f32
     of the shapes above (the C entry point takes raw pointers and cannot check
     them), else CandleMoeError."""
+    if _native is not None:
+        rc = _native.fp8(input, gate_q, up_q, down_q, gate_scale, up_scale, down_scale, routing_weights, expert_indices,
+                       output, num_experts, top_k, activation, moe_type)
+        if rc is not None:
+            return check(rc)
     import torch
 
     def bad(msg):
@@ -422,6 +456,11 @@ def fused_moe_packed(input, gate_packed, up_packed, down_packed, routing_weights
     down None. input / output [T, H] f16 or bf16, routing_weights [T, k] f32,
     expert_indices [T, k] u32/i32; every tensor contiguous, on input's device
     and of these shapes, else CandleMoeError."""
+    if _native is not None:
+        rc = _native.packed(input, gate_packed, up_packed, down_packed, routing_weights, expert_indices, output,
+                          num_experts, top_k, activation, moe_type)
+        if rc is not None:
+            return check(rc)
     import torch
 
     def bad(msg):
@@ -486,6 +525,13 @@ class FusedMoE:
         [E, I, H] (Qwen3, moe_type 0) or None (Nomic, moe_type 1);
         routing_weights [T, k] f32; expert_indices [T, k] u32.
         """
+        if _native is not None:
+            out = _native.forward(self.num_experts, self.num_selected_experts, self.activation, input, gate_weights,
+                                up_weights, down_weights, routing_weights, expert_indices, moe_type)
+            if type(out) is int:
+                return check(out)
+            if out is not None:
+                return out
         import torch
 
         out_shape = tuple(input.shape[:1]) + tuple(input.shape[1:2]) if input.dim() == 2 else (0, 0)
