@@ -1417,11 +1417,17 @@ int candle_moe_router_topk(const void* hidden, const void* router_weight, void* 
     if (((uintptr_t)hidden | (uintptr_t)router_weight) & 15)
         return cm::set_error(CANDLE_MOE_ERR_UNSUPPORTED, "router_topk: hidden and router_weight must be 16-byte aligned");
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    // small batches split K over workgroups, with f32 partials in the
-    // library-owned workspace of this (device, stream) (held while enqueuing,
+    // batches of few token tiles split K over workgroups, with f32 partials in
+    // the library-owned workspace of this (device, stream) (held while enqueuing,
     // as fused_moe does)
     // (after the workspace header, whose counters stay zero)
-    const size_t rneed = cm::router_ws_bytes(T, H, E, (int)dtype);
+    // A captured call of more than kRouterSplitTokens tokens runs in one pass:
+    // its graph then holds no pointer into a workspace that a later, larger call
+    // replaces.
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    const bool one_pass = T > cm::kRouterSplitTokens && cm::router_splits(T, H, E, (int)dtype) > 1 &&
+                          (hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone);
+    const size_t rneed = one_pass ? 0 : cm::router_ws_bytes(T, H, E, (int)dtype);
     const size_t need = rneed > 0 ? cm::kWsHeaderBytes + rneed : 0;
     hipError_t e = hipSuccess;
     if (need > 0) {
@@ -1430,12 +1436,13 @@ int candle_moe_router_topk(const void* hidden, const void* router_weight, void* 
         if (e != hipSuccess) return cm::hip_fail(e, "router_topk: hipGetDevice");
         std::lock_guard<std::mutex> lk(cm::g_ws_mu);
         cm::OwnedWs* w = cm::owned_ws_locked(dev, s, need, e, [] { return (size_t)0; });
-        if (!w) return cm::ws_fail("router_topk", need, e);
+        if (!w && T <= cm::kRouterSplitTokens) return cm::ws_fail("router_topk", need, e);
+        if (!w) (void)hipGetLastError();  // (no memory for it: one pass)
         e = cm::launch_router_topk(hidden, router_weight, (int)dtype, reinterpret_cast<float*>(topk_weight),
                                    reinterpret_cast<uint32_t*>(topk_indices),
                                    reinterpret_cast<uint32_t*>(token_expert_indices), T, H, E, k, s,
-                                   reinterpret_cast<float*>(static_cast<char*>(w->ptr) + cm::kWsHeaderBytes),
-                                   w->bytes - cm::kWsHeaderBytes);
+                                   w ? reinterpret_cast<float*>(static_cast<char*>(w->ptr) + cm::kWsHeaderBytes) : nullptr,
+                                   w ? w->bytes - cm::kWsHeaderBytes : 0);
     } else {
         e = cm::launch_router_topk(hidden, router_weight, (int)dtype, reinterpret_cast<float*>(topk_weight),
                                    reinterpret_cast<uint32_t*>(topk_indices),

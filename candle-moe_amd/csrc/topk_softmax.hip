@@ -921,11 +921,16 @@ __global__ __launch_bounds__(64) void router_topk_kernel(const void* __restrict_
 // and NB*KH waves, wave (c, h) computing the logits of experts 32c .. 32c+31
 // with v_mfma_f32_32x32x16 (A = token rows, B = weight rows, both
 // K-contiguous) over the k16 steps h*4/KH .. (h+1)*4/KH-1 of every K tile;
-// the waves with h = 0 issue the DMA.
-// K tiles of 64 reach LDS by buffer_load ... lds in an NST-stage ring, each
-// instruction covering 8 rows x 128 contiguous bytes (row loads straight
-// into the MFMA fragment registers touch 32 rows per instruction, which the
-// address unit serialises); rows past T or E and the K tail read as zeros.
+// all waves issue the DMA.
+// Stages of U K tiles of 64 reach LDS by buffer_load ... lds in an NST-stage
+// ring, each instruction covering 8 rows x 128 contiguous bytes (loads straight
+// into the MFMA fragment registers touch 16 rows or more per instruction, and a
+// CU takes a line per ~4 clocks: 16-row fragments, K split over the waves, no
+// LDS, 26.4 us at H=2048 E=128 T=4099); rows past T or E and the K tail read as
+// zeros. A stage's wait, barrier, LDS reads and products follow each other,
+// ~0.28 us whatever E: U = 2 halves their number. H=2048 E=128 T=4099 16.8 ->
+// 15.2 us, H=4096 E=64 T=4099 23.7 -> 18.4 (1.6 of it by all waves issuing the
+// DMA, not the h = 0 ones), H=768 E=40 T=700 8.2 -> 7.2.
 // Rows of a stage hold 8 16-byte chunks, chunk c of row r at a_swz(r, c)
 // (conflict-free fragment reads). The result layout puts expert 32c + l%32
 // of token 32m + 8(i/4) + 4(l/32) + i%4 in register i of block m of lane l;
@@ -937,7 +942,7 @@ __global__ __launch_bounds__(64) void router_topk_kernel(const void* __restrict_
 // tile runs K tiles [s*per, (s+1)*per) and stores each wave's f32 partial
 // logits (no rounding, no softmax) to part[s*KH + kh][t][e], for
 // topk_partials_kernel to sum in split order.
-template <int DT, int NB, int MT, int NST, int KH, bool PART = false>
+template <int DT, int NB, int MT, int U, int NST, int KH, bool PART = false>
 __global__ __launch_bounds__(64 * NB * KH) void router_mfma_kernel(const void* __restrict__ xin,
                                                               const void* __restrict__ win,
                                                               float* __restrict__ wout, uint32_t* __restrict__ iout,
@@ -948,10 +953,15 @@ __global__ __launch_bounds__(64 * NB * KH) void router_mfma_kernel(const void* _
     typedef typename Elem<DT>::storage S;
     constexpr int TM = 32 * MT;                   // tokens per workgroup
     constexpr int EW = 32 * NB;                   // weight rows (experts, padded)
-    constexpr int STAGE = (TM + EW) * 128;        // one K tile of 64: 128 bytes per row
+    constexpr int SUB = (TM + EW) * 128;          // one K tile of 64: 128 bytes per row
+    constexpr int STAGE = U * SUB;
     constexpr int INS = STAGE / 1024;             // DMA instructions per stage (8 rows each)
-    constexpr int LOADS = INS / NB;               // per wave
-    static_assert(LOADS * NB == INS && LOADS * (NST - 2) < 64, "router stage split");
+    // all waves issue, instruction NW*i + wave of a stage each: the first REM
+    // waves one more (a wave's DMA instructions follow each other at ~110
+    // clocks)
+    constexpr int NWV = NB * KH;
+    constexpr int LMIN = INS / NWV, REM = INS % NWV, LOADS = LMIN + (REM ? 1 : 0);
+    static_assert(LMIN >= 1 && LOADS * (NST - 2) < 64, "router stage split");
     static_assert(KH * MT * NB * 16 * 64 * 4 <= NST * STAGE, "softmax exchange fits the ring");
     static_assert(KH == 1 || KH == 2, "K halves");
     __shared__ __attribute__((aligned(1024))) char smem[NST * STAGE];
@@ -965,33 +975,37 @@ __global__ __launch_bounds__(64 * NB * KH) void router_mfma_kernel(const void* _
     const i32x4 rw = make_rsrc(win, (long long)E * H * 2);
     const uint32_t sbase = __builtin_amdgcn_readfirstlane(lds_addr(smem));
 
-    // per-lane source offsets of this wave's LOADS instructions (instruction
-    // q = NB*i + wave of the stage: rows 8q .. 8q+7, token rows first), the K
-    // position of a full tile in the SGPR offset
+    // per-lane source offsets of this wave's instructions (instruction q of the
+    // stage: rows 8q .. 8q+7, token rows first), the K position of a full tile
+    // in the SGPR offset
     uint32_t off[LOADS];
-    int chunk_k[LOADS];
+    int chunk_k[LOADS];  // (relative to the stage's first K tile)
     bool is_x[LOADS];
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) {
-        const int q = NB * i + cb;
-        const int row = 8 * q + lane / 8;  // row of the stage
+        const int q = (NWV * i + wave) % (SUB / 1024), u = (NWV * i + wave) / (SUB / 1024);
+        const int row = 8 * q + lane / 8;  // row of the K tile
         const int c = a_swz<8>(row, lane % 8);
-        chunk_k[i] = 8 * c;
+        chunk_k[i] = 64 * u + 8 * c;
         is_x[i] = 8 * q < TM;  // whole instructions: TM is a multiple of 8 (wave-uniform)
-        off[i] = is_x[i] ? ((uint32_t)row * (uint32_t)H + 8u * c) * 2u
-                         : ((uint32_t)(row - TM) * (uint32_t)H + 8u * c) * 2u;  // rows >= rows / E: past the resource
+        off[i] = ((uint32_t)(is_x[i] ? row : row - TM) * (uint32_t)H + (uint32_t)chunk_k[i]) *
+                 2u;  // rows >= rows / E: past the resource
     }
+    const bool more = wave < REM;
     const int nk_all = (H + 63) / 64;
     const int per = (nk_all + ks - 1) / ks;
     const int kt_lo = PART ? min(nk_all, split * per) : 0;
     const int nk = PART ? min(nk_all, kt_lo + per) - kt_lo : nk_all;  // this split's K tiles (may be 0)
+    const int k_end = PART ? min(H, (kt_lo + nk) * 64) : H;
+    const int ns = (nk + U - 1) / U;  // stages
     auto issue = [&](int stage, int k0) {
         const uint32_t sl = sbase + stage * STAGE;
-        const bool full = k0 + 64 <= H;
+        const bool full = k0 + 64 * U <= k_end;
 #pragma unroll
         for (int i = 0; i < LOADS; ++i) {
-            const uint32_t v = (full || k0 + chunk_k[i] < H) ? off[i] : kOob;
-            dma16s(is_x[i] ? rx : rw, sl + (NB * i + cb) * 1024, v, (uint32_t)k0 * 2u);
+            if (i == LMIN && !more) break;  // (wave-uniform)
+            const uint32_t v = (full || k0 + chunk_k[i] < k_end) ? off[i] : kOob;
+            dma16s(is_x[i] ? rx : rw, sl + (NWV * i + wave) * 1024, v, (uint32_t)k0 * 2u);
         }
     };
 
@@ -1001,27 +1015,23 @@ __global__ __launch_bounds__(64 * NB * KH) void router_mfma_kernel(const void* _
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[m][i] = 0.f;
     const int lr = lane & 31, lh = lane >> 5;
-    const bool dma = kh == 0;
 #pragma unroll
     for (int s = 0; s < NST - 1; ++s)
-        if (dma && s < nk) issue(s, (kt_lo + s) * 64);
-    for (int kt = 0; kt < nk; ++kt) {
-        // this wave's DMA of tile kt (NST-2 newer tiles may stay in flight),
+        if (s < ns) issue(s, (kt_lo + s * U) * 64);
+    for (int kt = 0; kt < ns; ++kt) {
+        // this wave's DMA of stage kt (NST-2 newer stages may stay in flight),
         // then the barrier makes every wave's part visible and frees slot kt-1
-        const int newer = min(NST - 2, nk - 1 - kt);
-        if (newer >= 4) wait_vm<4 * LOADS>();
-        else if (newer == 3) wait_vm<3 * LOADS>();
-        else if (newer == 2) wait_vm<2 * LOADS>();
-        else if (newer == 1) wait_vm<LOADS>();
-        else wait_vm<0>();
+        const int newer = min(NST - 2, ns - 1 - kt);
+        if (more) wait_stage<LOADS, NST - 2>(newer);
+        else wait_stage<LMIN, NST - 2>(newer);
         wait_lgkm0();
         block_barrier();
-        if (dma && kt + NST - 1 < nk) issue((kt + NST - 1) % NST, (kt_lo + kt + NST - 1) * 64);
-        const char* sx = smem + (kt % NST) * STAGE;
-        const char* sw = sx + TM * 128;
+        if (kt + NST - 1 < ns) issue((kt + NST - 1) % NST, (kt_lo + (kt + NST - 1) * U) * 64);
 #pragma unroll
-        for (int s4 = 0; s4 < 4 / KH; ++s4) {
-            const int st = kh * (4 / KH) + s4;
+        for (int s4 = 0; s4 < U * (4 / KH); ++s4) {
+            const char* sx = smem + (kt % NST) * STAGE + s4 / (4 / KH) * SUB;
+            const char* sw = sx + TM * 128;
+            const int st = kh * (4 / KH) + s4 % (4 / KH);
             const int c = 2 * st + lh;
             const int wr = 32 * cb + lr;  // weight row; stage row TM + wr (the swizzle's row)
             const u32x4 b = *reinterpret_cast<const u32x4*>(sw + wr * 128 + a_swz<8>(TM + wr, c) * 16);
@@ -1100,21 +1110,26 @@ __global__ __launch_bounds__(64 * NB * KH) void router_mfma_kernel(const void* _
     }
 }
 
-// Small batches (at most kRouterSplitTiles tiles of 32 tokens): K split over
+// Small batches (up to kRouterSplitTokens): K split over
 // ks workgroups per tile (aiming at ~64 workgroups, at least 2 K tiles each,
 // at most kRouterMaxSlots splits), one f32 partial per split in the caller's
 // workspace (the split's waves each cover all of its K tiles), then the
 // softmax / top-k summing them (two launches instead of one workgroup per
-// tile streaming the whole router weight).
-constexpr int kRouterSplitTiles = 8;
+// tile streaming the whole router weight). Larger batches are split while the
+// tiles leave CUs for it (256 workgroups) and each workgroup is spared at least
+// kRouterSplitSaves K tiles of ~0.25 us, which pays for the second launch and
+// the partials: H=2048 E=128 T=257 / 1000 / 2000 14.6 / 14.8 / 14.9 -> 11.1 /
+// 13.0 / 13.4 us, H=4096 E=64 T=1000 17.9 -> 13.0; below the line H=2048 T=4096
+// (16 spared) 15.2 against 15.6 us split, H=768 E=40 T=700 (10) 7.2 against 10.2.
+// Those run in one pass under graph capture and without the workspace.
+constexpr int kRouterSplitSaves = 24;
 int router_splits(int T, int H, int E, int dtype) {
     if (dtype == kF32 || E <= 32 || E > 128) return 1;
     const long long tiles = ((long long)T + 31) / 32;
-    if (tiles > kRouterSplitTiles) return 1;
     const int nk = (H + 63) / 64;
-    int ks = (int)(64 / tiles);
-    ks = std::min(ks, std::min(kRouterMaxSlots, nk / 2));
-    return ks >= 2 ? ks : 1;
+    int ks = (int)std::min<long long>((T <= kRouterSplitTokens ? 64 : 256) / tiles, std::min(kRouterMaxSlots, nk / 2));
+    if (ks < 2 || (T > kRouterSplitTokens && nk - (nk + ks - 1) / ks < kRouterSplitSaves)) return 1;
+    return ks;
 }
 size_t router_ws_bytes(int T, int H, int E, int dtype) {
     const int ks = router_splits(T, H, E, dtype);
@@ -1125,7 +1140,7 @@ template <int DT, int NB>
 static hipError_t launch_router_split(const void* x, const void* w, float* wo, uint32_t* io, uint32_t* eo, int T,
                                       int H, int E, int k, int ks, float* part, hipStream_t stream) {
     const long long grid = ((long long)T + 31) / 32 * ks;
-    hipLaunchKernelGGL((router_mfma_kernel<DT, NB, 1, 6, 1, true>), dim3((unsigned)grid), dim3(64 * NB), 0, stream,
+    hipLaunchKernelGGL((router_mfma_kernel<DT, NB, 1, 2, 3, 1, true>), dim3((unsigned)grid), dim3(64 * NB), 0, stream,
                        x, w, wo, io, eo, T, H, E, k, part, ks);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
@@ -1143,18 +1158,21 @@ static hipError_t launch_router_split(const void* x, const void* w, float* wo, u
 template <int DT, int NB>
 static hipError_t launch_router_mfma(const void* x, const void* w, float* wo, uint32_t* io, uint32_t* eo, int T,
                                      int H, int E, int k, hipStream_t stream) {
-    // 64 tokens per workgroup (each weight tile serves twice the rows) once
-    // that still gives >= 256 workgroups, 3 stages (72 KB: two workgroups per
-    // CU, 85 -> 63 us at T=32768, E=128 against 5 stages); else 32 tokens and
-    // 6 stages (the one workgroup of a CU keeps more of the weight in flight)
-    if ((long long)T >= 256LL * 64) {
+    // 64 tokens per workgroup (each weight tile serves twice the rows), 3
+    // stages of one K tile (72 KB: two workgroups per CU, 85 -> 63 us at
+    // T=32768, E=128 against 5 stages), once the 32-token tiles of E > 64 (120
+    // KB) would take a second round on 256 CUs (T=12000 29.3 -> 24.5 us), or
+    // there are 256 of these (E <= 64: two workgroups of 72 KB per CU either
+    // way, T=9000 H=768 E=40 11.6 against 9.3 us below it); else 32 tokens and
+    // 3 stages of two K tiles
+    if ((long long)T > (NB > 2 ? 256LL * 32 : 256LL * 64 - 1)) {
         const long long grid = ((long long)T + 63) / 64;
         if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
-        hipLaunchKernelGGL((router_mfma_kernel<DT, NB, 2, 3, 2>), dim3((unsigned)grid), dim3(128 * NB), 0, stream, x, w,
+        hipLaunchKernelGGL((router_mfma_kernel<DT, NB, 2, 1, 3, 2>), dim3((unsigned)grid), dim3(128 * NB), 0, stream, x, w,
                            wo, io, eo, T, H, E, k);
     } else {
         const long long grid = ((long long)T + 31) / 32;
-        hipLaunchKernelGGL((router_mfma_kernel<DT, NB, 1, 6, 2>), dim3((unsigned)grid), dim3(128 * NB), 0, stream, x, w,
+        hipLaunchKernelGGL((router_mfma_kernel<DT, NB, 1, 2, 3, 2>), dim3((unsigned)grid), dim3(128 * NB), 0, stream, x, w,
                            wo, io, eo, T, H, E, k);
     }
     return hipGetLastError();
