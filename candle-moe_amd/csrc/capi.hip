@@ -322,7 +322,8 @@ static bool dec_gemv_fits(const Problem& p) {
 // 5.9 TB/s), so slices let 128-column blocks (256-byte runs) fill the
 // device. Bounds: at least kDecMinSteps steps of 32 k per wave (kp waves
 // share a slice of one tensor) and f32 partials of at most kDecPartBytes.
-// Used where the weight stream is at least kDecSliceBytes (check_problem).
+// Used where the weight stream is at least kDecSliceBytes, or in few long blocks
+// (check_problem).
 constexpr int kDecMinSteps = 1;
 constexpr double kDecPartBytes = 16.0 * 1024 * 1024;
 constexpr double kDecSliceBytes = 128.0 * 1024 * 1024;
@@ -626,7 +627,8 @@ static int check_problem(int T, int H, int I, int E, int k, int act, uint32_t mo
     p.dec_ks1 = p.dec_ks2 = 1;
     if (p.cfg == kDecGemv) {
         // K slices for the gate/up (fc1) GEMM only where they paid: few
-        // column blocks of 128 and a large weight stream. Measured steps
+        // column blocks of 128 and a large weight stream, or few and long
+        // blocks (below). Measured steps
         // (router + forward, graph-replayed, cold bf16 weights), sliced
         // against not: Qwen3 T=8 / 64 65.1 / 80.1 against 73.3 / 84.1 us;
         // Qwen3-30B-A3B T=1 / 16 29.6 / 83.4 against 29.0 / 78.4 us, Nomic
@@ -641,7 +643,15 @@ static int check_problem(int T, int H, int I, int E, int k, int act, uint32_t mo
         // its items would leave CUs idle (Nomic's fc2 has 96 of them)
         const int cols = p.dtype == kF32 ? 64 : 128;
         const double part = p.dtype == kF32 ? kDecPartBytesF32 : kDecPartBytes;
-        if (groups * cdiv(I, cols) < 256 && wbytes >= kDecSliceBytes)
+        // 16-bit also where the GEMM's 64-column blocks are few (a quarter of
+        // the CUs) and stream 1 MiB each: one or two tokens over large experts.
+        // Steps unsliced / sliced: Qwen3 T=1 36.0 / 27.8 us (pre-packed 38.0 /
+        // 34.3), H 8192 I 2048 k 1 T=1 85.6 / 37.9, H 4096 I 512 E 128 k 8 T=1
+        // 51.0 / 32.2. At 96 blocks (Qwen3 T=2) 57.9 / 43.0, but pre-packed,
+        // which takes the same slices to give the same bits, 48.2 / 51.1.
+        const bool few = p.dtype != kF32 && !fp8 && groups * cdiv(I, 64) <= 64 &&
+                         (long long)(q3 ? 2 : 1) * H * 128 >= (1 << 20);
+        if (groups * cdiv(I, cols) < 256 && (wbytes >= kDecSliceBytes || few))
             p.dec_ks1 = dec_slices(P, I, H, q3 ? 2 : 4, q3 ? 2 : 1, part);
         if (p.dtype == kF32 && groups * cdiv(H, cols) < 256) p.dec_ks2 = dec_slices(P, H, I, 4, 1, part);
     }
