@@ -1122,6 +1122,10 @@ __global__ __launch_bounds__(64 * NB * KH) void router_mfma_kernel(const void* _
 // 13.0 / 13.4 us, H=4096 E=64 T=1000 17.9 -> 13.0; below the line H=2048 T=4096
 // (16 spared) 15.2 against 15.6 us split, H=768 E=40 T=700 (10) 7.2 against 10.2.
 // Those run in one pass under graph capture and without the workspace.
+// Shorter running sums are no further from 64 bits: of normal rows, those whose
+// outputs move because a logit rounds to the other 16-bit neighbour number 399
+// split, 494 in one pass (24 inputs each of T=3283 and 2000 H=4096 E=64, T=1000
+// H=2048 E=128, T=700 H=2880 E=128); a single input can go either way.
 constexpr int kRouterSplitSaves = 24;
 int router_splits(int T, int H, int E, int dtype) {
     if (dtype == kF32 || E <= 32 || E > 128) return 1;
