@@ -1041,12 +1041,18 @@ static int check_ptrs(const Problem& p, const void* x, const void* gate, const v
 // ordered after the previous one on that stream; the lock is held while a
 // call enqueues its kernels, so two host threads on one stream never
 // interleave their launches over the shared buffer. A grown buffer's old
-// allocation is released with hipFreeAsync on its own stream.
+// allocation is released with hipFreeAsync on its own stream, unless a call
+// was captured into a graph while it was the stream's buffer: the graph's
+// kernels keep its address, whatever larger call the stream sees later, so it
+// is kept (`replaced`) until the workspaces are trimmed. Buffers grow by half at
+// least, so those of a stream hold at most twice its current one's bytes.
 struct OwnedWs {
     int device;
     hipStream_t stream;
     void* ptr;
     size_t bytes;
+    bool captured;  // a graph may hold ptr
+    std::vector<void*> replaced;
 };
 static std::mutex g_ws_mu;
 static std::vector<OwnedWs> g_ws;
@@ -1056,15 +1062,24 @@ static std::vector<OwnedWs> g_ws;
 // allocation node to the caller's graph, memory the graph owns and releases
 // when it is destroyed, while this table would keep handing it out.
 // reserve: bytes to allocate at least, asked for when the workspace grows.
+static bool is_capturing(hipStream_t s) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cs) == hipSuccess) return cs != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return false;
+}
 template <class F>
 static OwnedWs* owned_ws_locked(int dev, hipStream_t s, size_t need, hipError_t& err, F&& reserve) {
     err = hipSuccess;
     OwnedWs* w = nullptr;
     for (auto& e : g_ws)
         if (e.device == dev && e.stream == s) w = &e;
-    if (w && w->bytes >= need) return w;
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone) {
+    const bool capturing = is_capturing(s);
+    if (w && w->bytes >= need) {
+        w->captured = w->captured || capturing;
+        return w;
+    }
+    if (capturing) {
         err = hipErrorStreamCaptureUnsupported;
         return nullptr;
     }
@@ -1083,12 +1098,14 @@ static OwnedWs* owned_ws_locked(int dev, hipStream_t s, size_t need, hipError_t&
         return nullptr;
     }
     if (w) {
-        if (w->ptr) (void)hipFreeAsync(w->ptr, s);
+        if (w->captured) w->replaced.push_back(w->ptr);
+        else if (w->ptr) (void)hipFreeAsync(w->ptr, s);
         w->ptr = mem;
         w->bytes = want;
+        w->captured = false;
         return w;
     }
-    g_ws.push_back(OwnedWs{dev, s, mem, want});
+    g_ws.push_back(OwnedWs{dev, s, mem, want, false, {}});
     return &g_ws.back();
 }
 
@@ -1110,10 +1127,12 @@ int trim_owned_workspaces() {
     // may have been destroyed since its last call (hipFree waits for the
     // device instead)
     for (auto& e : g_ws) {
-        if (!e.ptr) continue;
         if (e.device != cur) (void)hipSetDevice(e.device);
-        const hipError_t r = hipFree(e.ptr);
-        if (first == hipSuccess) first = r;
+        e.replaced.push_back(e.ptr);
+        for (void* q : e.replaced) {
+            const hipError_t r = q ? hipFree(q) : hipSuccess;
+            if (first == hipSuccess) first = r;
+        }
         if (e.device != cur && cur >= 0) (void)hipSetDevice(cur);
     }
     g_ws.clear();

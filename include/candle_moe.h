@@ -73,7 +73,9 @@ void topk_softmax(const void* gating_output, void* topk_weight, void* topk_indic
  * The workspace is library-owned: one buffer per (device, stream), allocated
  * stream-ordered (hipMallocAsync on `stream`) on first use, grown when a call
  * needs more and kept for the next call on that stream;
- * candle_moe_trim_workspaces releases them. No host synchronisation. A stream
+ * candle_moe_trim_workspaces releases them. No host synchronisation. A buffer
+ * that captured calls use stays allocated when a larger call replaces it, until
+ * the workspaces are trimmed: their graphs stay valid until then. A stream
  * being captured into a graph gets no new or larger workspace (the graph
  * would own that memory): such a call fails with CANDLE_MOE_ERR_WORKSPACE
  * before enqueuing anything, so make one call of the largest size on the
