@@ -1450,12 +1450,10 @@ int candle_moe_router_topk(const void* hidden, const void* router_weight, void* 
     // the library-owned workspace of this (device, stream) (held while enqueuing,
     // as fused_moe does)
     // (after the workspace header, whose counters stay zero)
-    // A captured call of more than kRouterSplitTokens tokens runs in one pass:
-    // its graph then holds no pointer into a workspace that a later, larger call
-    // replaces.
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    const bool one_pass = T > cm::kRouterSplitTokens && cm::router_splits(T, H, E, (int)dtype) > 1 &&
-                          (hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone);
+    // A captured call of more than kRouterSplitTokens tokens needs no workspace
+    // (its stream may have none): the same sums in one pass.
+    const bool one_pass =
+        T > cm::kRouterSplitTokens && cm::router_splits(T, H, E, (int)dtype) > 1 && cm::is_capturing(s);
     const size_t rneed = one_pass ? 0 : cm::router_ws_bytes(T, H, E, (int)dtype);
     const size_t need = rneed > 0 ? cm::kWsHeaderBytes + rneed : 0;
     hipError_t e = hipSuccess;

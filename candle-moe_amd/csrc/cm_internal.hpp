@@ -9,7 +9,8 @@ namespace cm {
 
 // ---------------------------------------------------------------- router
 // part / part_bytes: workspace of router_ws_bytes() for the K-split form
-// (router_splits() > 1); without it one workgroup per tile.
+// (router_splits() > 1); without it one workgroup per tile adds the same K
+// ranges up, with the same results bit for bit.
 hipError_t launch_router_topk(const void* x, const void* w, int dtype, float* wo, uint32_t* io, uint32_t* eo, int T,
                               int H, int E, int k, hipStream_t stream, float* part = nullptr,
                               size_t part_bytes = 0);

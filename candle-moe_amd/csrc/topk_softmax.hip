@@ -938,11 +938,19 @@ __global__ __launch_bounds__(64) void router_topk_kernel(const void* __restrict_
 // order) so that each holds whole tokens for the softmax over 32-lane groups
 // (VPT = NB experts per lane, stride 32); KH = 2 halves the rows each wave
 // ranks, whose top-k passes dominate small batches.
-// PART (small batches): the grid is token tiles x ks K splits; split s of a
+// kRouterPart (few token tiles): the grid is token tiles x ks K splits; split s of a
 // tile runs K tiles [s*per, (s+1)*per) and stores each wave's f32 partial
 // logits (no rounding, no softmax) to part[s*KH + kh][t][e], for
 // topk_partials_kernel to sum in split order.
-template <int DT, int NB, int MT, int U, int NST, int KH, bool PART = false>
+// kRouterSums: the same sums without the workspace, bit for bit: one workgroup
+// per tile runs the ks K ranges two at a time, wave (c, h) the h-th of a pair
+// (the two K tiles of a stage come from the two ranges); the waves with h = 0
+// add the ranges' sums up in order, the others' through LDS one stage later,
+// and the softmax is taken as in topk_partials_kernel (same lane groups, same
+// rows per wave, whose rows share the choice of the exact softmax). For calls
+// that may not keep a workspace (graph capture).
+enum { kRouterWhole, kRouterPart, kRouterSums };
+template <int DT, int NB, int MT, int U, int NST, int KH, int FORM = kRouterWhole>
 __global__ __launch_bounds__(64 * NB * KH) void router_mfma_kernel(const void* __restrict__ xin,
                                                               const void* __restrict__ win,
                                                               float* __restrict__ wout, uint32_t* __restrict__ iout,
@@ -951,6 +959,8 @@ __global__ __launch_bounds__(64 * NB * KH) void router_mfma_kernel(const void* _
                                                               int ks = 1) {
     using namespace lds;
     typedef typename Elem<DT>::storage S;
+    constexpr bool PART = FORM == kRouterPart, SUMS = FORM == kRouterSums;
+    static_assert(!SUMS || (MT == 1 && KH == 2 && U == 2), "split sums: a K range per wave row");
     constexpr int TM = 32 * MT;                   // tokens per workgroup
     constexpr int EW = 32 * NB;                   // weight rows (experts, padded)
     constexpr int SUB = (TM + EW) * 128;          // one K tile of 64: 128 bytes per row
@@ -978,6 +988,9 @@ __global__ __launch_bounds__(64 * NB * KH) void router_mfma_kernel(const void* _
     // per-lane source offsets of this wave's instructions (instruction q of the
     // stage: rows 8q .. 8q+7, token rows first), the K position of a full tile
     // in the SGPR offset
+    const int nk_all = (H + 63) / 64;
+    const int per = FORM == kRouterWhole ? nk_all : (nk_all + ks - 1) / ks;  // (SUMS: at least 2)
+    const int u_k = 64 * (SUMS ? per : 1);  // from one K tile of a stage to the next
     uint32_t off[LOADS];
     int chunk_k[LOADS];  // (relative to the stage's first K tile)
     bool is_x[LOADS];
@@ -986,21 +999,29 @@ __global__ __launch_bounds__(64 * NB * KH) void router_mfma_kernel(const void* _
         const int q = (NWV * i + wave) % (SUB / 1024), u = (NWV * i + wave) / (SUB / 1024);
         const int row = 8 * q + lane / 8;  // row of the K tile
         const int c = a_swz<8>(row, lane % 8);
-        chunk_k[i] = 64 * u + 8 * c;
+        chunk_k[i] = u_k * u + 8 * c;
         is_x[i] = 8 * q < TM;  // whole instructions: TM is a multiple of 8 (wave-uniform)
         off[i] = ((uint32_t)(is_x[i] ? row : row - TM) * (uint32_t)H + (uint32_t)chunk_k[i]) *
                  2u;  // rows >= rows / E: past the resource
     }
     const bool more = wave < REM;
-    const int nk_all = (H + 63) / 64;
-    const int per = (nk_all + ks - 1) / ks;
     const int kt_lo = PART ? min(nk_all, split * per) : 0;
     const int nk = PART ? min(nk_all, kt_lo + per) - kt_lo : nk_all;  // this split's K tiles (may be 0)
     const int k_end = PART ? min(H, (kt_lo + nk) * 64) : H;
-    const int ns = (nk + U - 1) / U;  // stages
-    auto issue = [&](int stage, int k0) {
+    // stages (SUMS: per of them for each pair of ranges, fewer where the last
+    // range is alone and short)
+    const int nr = (nk_all + per - 1) / per;
+    const int ns = SUMS ? nr / 2 * per + (nr % 2) * (nk_all - (nr - 1) * per) : (nk + U - 1) / U;
+    int is_k0 = kt_lo * 64, is_j = 0;  // the stage issued next: its K, its place in the pair of ranges
+    auto issue = [&](int stage) {
+        const int k0 = is_k0;
+        is_k0 += SUMS ? 64 : 64 * U;
+        if (SUMS && ++is_j == per) {
+            is_j = 0;
+            is_k0 += u_k;
+        }
         const uint32_t sl = sbase + stage * STAGE;
-        const bool full = k0 + 64 * U <= k_end;
+        const bool full = k0 + (U - 1) * u_k + 64 <= k_end;
 #pragma unroll
         for (int i = 0; i < LOADS; ++i) {
             if (i == LMIN && !more) break;  // (wave-uniform)
@@ -1014,10 +1035,38 @@ __global__ __launch_bounds__(64 * NB * KH) void router_mfma_kernel(const void* _
     for (int m = 0; m < MT; ++m)
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[m][i] = 0.f;
+    // SUMS: the ranges' sums added up so far, the waves' exchange (h = 1 to 0),
+    // whether it holds a sum to be added, this stage's place in its pair
+    f32x16 tot;
+    if constexpr (SUMS) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) tot[i] = 0.f;
+    }
+    __shared__ f32x4 s_x[SUMS ? NB * 4 * 64 : 1];
+    f32x4* const xch = s_x + (SUMS ? cb * 4 * 64 + lane : 0);
+    auto add = [&](const f32x4* from) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const f32x4 v = from[q * 64];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) tot[4 * q + j] += v[j];
+        }
+    };
+    auto give = [&](f32x4* to) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            to[q * 64] = f32x4{acc[0][4 * q], acc[0][4 * q + 1], acc[0][4 * q + 2], acc[0][4 * q + 3]};
+    };
+    auto own = [&]() {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) tot[i] += acc[0][i];
+    };
+    bool pending = false;
+    int pair_j = 0;
     const int lr = lane & 31, lh = lane >> 5;
 #pragma unroll
     for (int s = 0; s < NST - 1; ++s)
-        if (s < ns) issue(s, (kt_lo + s * U) * 64);
+        if (s < ns) issue(s);
     for (int kt = 0; kt < ns; ++kt) {
         // this wave's DMA of stage kt (NST-2 newer stages may stay in flight),
         // then the barrier makes every wave's part visible and frees slot kt-1
@@ -1026,12 +1075,24 @@ __global__ __launch_bounds__(64 * NB * KH) void router_mfma_kernel(const void* _
         else wait_stage<LMIN, NST - 2>(newer);
         wait_lgkm0();
         block_barrier();
-        if (kt + NST - 1 < ns) issue((kt + NST - 1) % NST, (kt_lo + (kt + NST - 1) * U) * 64);
+        if (kt + NST - 1 < ns) issue((kt + NST - 1) % NST);
+        if constexpr (SUMS) {
+            // (written a barrier ago; the next write is a barrier away: per >= 2)
+            if (pending && kh == 0) add(xch);
+            pending = kt > 0 && pair_j == 0;  // a pair of ranges is done
+            if (pending) {
+                if (kh == 0) own();
+                else give(xch);
+#pragma unroll
+                for (int i = 0; i < 16; ++i) acc[0][i] = 0.f;
+            }
+            pair_j = pair_j + 1 == per ? 0 : pair_j + 1;
+        }
 #pragma unroll
         for (int s4 = 0; s4 < U * (4 / KH); ++s4) {
-            const char* sx = smem + (kt % NST) * STAGE + s4 / (4 / KH) * SUB;
+            const char* sx = smem + (kt % NST) * STAGE + (SUMS ? kh : s4 / (4 / KH)) * SUB;
             const char* sw = sx + TM * 128;
-            const int st = kh * (4 / KH) + s4 % (4 / KH);
+            const int st = SUMS ? s4 : kh * (4 / KH) + s4 % (4 / KH);
             const int c = 2 * st + lh;
             const int wr = 32 * cb + lr;  // weight row; stage row TM + wr (the swizzle's row)
             const u32x4 b = *reinterpret_cast<const u32x4*>(sw + wr * 128 + a_swz<8>(TM + wr, c) * 16);
@@ -1057,10 +1118,44 @@ __global__ __launch_bounds__(64 * NB * KH) void router_mfma_kernel(const void* _
             }
         return;
     }
-    // exchange through LDS (the ring is free after the barrier):
-    // red[kh][m][c][i][lane]
     wait_lgkm0();
     __syncthreads();
+    if constexpr (SUMS) {
+        // the last pair's sums, then whole logit rows through LDS (the ring is
+        // free after the barrier) and the rows' lane groups as in
+        // topk_partials_kernel
+        constexpr int VPT = 8, LPR = EW / VPT, RS = EW + 4, GROUPS = 64 * NB * KH / LPR;
+        static_assert(TM * RS * 4 + GROUPS * EW * 4 + NB * 4096 <= NST * STAGE && TM == GROUPS,
+                      "logit rows fit the ring");
+        float* lrow = reinterpret_cast<float*>(smem);
+        float* s_p = lrow + TM * RS;
+        f32x4* last = reinterpret_cast<f32x4*>(s_p + GROUPS * EW) + cb * 4 * 64 + lane;
+        if (kh == 1) {
+            give(last);
+        } else {
+            if (pending) add(xch);
+            own();
+        }
+        __syncthreads();
+        if (kh == 0) {
+            add(last);
+#pragma unroll
+            for (int i = 0; i < 16; ++i) lrow[(8 * (i / 4) + 4 * lh + (i % 4)) * RS + 32 * cb + lr] = tot[i];
+        }
+        __syncthreads();
+        const int g = threadIdx.x % LPR, grp = threadIdx.x / LPR, e0 = VPT * g;
+        const long long row = t0 + grp;
+        const bool valid = row < T;
+        const float* src = lrow + (int)((valid ? row : (long long)T - 1) - t0) * RS + e0;
+        float x[VPT];
+#pragma unroll
+        for (int j = 0; j < VPT; ++j)
+            x[j] = e0 + j < E ? Elem<DT>::to_f32(Elem<DT>::from_f32(src[j])) : -__builtin_inff();
+        softmax_topk_group<VPT, LPR, kF32, 1, true>(x, e0, g, E, k, T, row, valid, wout, iout, eiout, s_p + grp * EW);
+        return;
+    }
+    // exchange through LDS (the ring is free after the barrier):
+    // red[kh][m][c][i][lane]
     float* red = reinterpret_cast<float*>(smem);
 #pragma unroll
     for (int m = 0; m < MT; ++m)
@@ -1121,7 +1216,11 @@ __global__ __launch_bounds__(64 * NB * KH) void router_mfma_kernel(const void* _
 // the partials: H=2048 E=128 T=257 / 1000 / 2000 14.6 / 14.8 / 14.9 -> 11.1 /
 // 13.0 / 13.4 us, H=4096 E=64 T=1000 17.9 -> 13.0; below the line H=2048 T=4096
 // (16 spared) 15.2 against 15.6 us split, H=768 E=40 T=700 (10) 7.2 against 10.2.
-// Those run in one pass under graph capture and without the workspace.
+// Those add the same K ranges up in one workgroup per tile under graph capture
+// and without the workspace (kRouterSums), with the same bits: graph-replayed,
+// T=257 / 1000 / 2000 H=2048 E=128, T=1000 H=4096 E=40 19.6 / 20.9 / 17.9 / 23.8
+// us, where kRouterWhole, which rounds otherwise, takes 19.3 / 19.4 / 19.6 / 20.9
+// (launching a graph is about 5 us of each).
 // Shorter running sums are no further from 64 bits: of normal rows, those whose
 // outputs move because a logit rounds to the other 16-bit neighbour number 399
 // split, 494 in one pass (24 inputs each of T=3283 and 2000 H=4096 E=64, T=1000
@@ -1143,8 +1242,13 @@ size_t router_ws_bytes(int T, int H, int E, int dtype) {
 template <int DT, int NB>
 static hipError_t launch_router_split(const void* x, const void* w, float* wo, uint32_t* io, uint32_t* eo, int T,
                                       int H, int E, int k, int ks, float* part, hipStream_t stream) {
-    const long long grid = ((long long)T + 31) / 32 * ks;
-    hipLaunchKernelGGL((router_mfma_kernel<DT, NB, 1, 2, 3, 1, true>), dim3((unsigned)grid), dim3(64 * NB), 0, stream,
+    const long long tiles = ((long long)T + 31) / 32, grid = tiles * ks;
+    if (!part) {
+        hipLaunchKernelGGL((router_mfma_kernel<DT, NB, 1, 2, 3, 2, kRouterSums>), dim3((unsigned)tiles), dim3(128 * NB),
+                           0, stream, x, w, wo, io, eo, T, H, E, k, nullptr, ks);
+        return hipGetLastError();
+    }
+    hipLaunchKernelGGL((router_mfma_kernel<DT, NB, 1, 2, 3, 1, kRouterPart>), dim3((unsigned)grid), dim3(64 * NB), 0, stream,
                        x, w, wo, io, eo, T, H, E, k, part, ks);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
@@ -1215,7 +1319,8 @@ hipError_t launch_router_topk(const void* x, const void* w, int dtype, float* wo
                               int H, int E, int k, hipStream_t stream, float* part, size_t part_bytes) {
     if (T == 0) return hipSuccess;
     const int ks = router_splits(T, H, E, dtype);
-    if (ks > 1 && part && part_bytes >= router_ws_bytes(T, H, E, dtype)) {
+    if (ks > 1) {
+        if (part_bytes < router_ws_bytes(T, H, E, dtype)) part = nullptr;
         if (dtype == kBF16)
             return E <= 64 ? launch_router_split<kBF16, 2>(x, w, wo, io, eo, T, H, E, k, ks, part, stream)
                            : launch_router_split<kBF16, 4>(x, w, wo, io, eo, T, H, E, k, ks, part, stream);

@@ -239,8 +239,9 @@ int candle_moe_fused_moe_path_ex(int num_tokens, int hidden_dim, int intermediat
  * weight stream over workgroups, with f32 partial logits in the library's
  * per-stream workspace (the one fused_moe keeps; allocated on first use,
  * never while the stream is being captured: see fused_moe). So do larger ones
- * of few token tiles and a large hidden_dim, but in one pass while the stream is
- * being captured or where there is no memory for the workspace. */
+ * of few token tiles and a large hidden_dim, but without the workspace while the
+ * stream is being captured or where there is no memory for it: one workgroup per
+ * tile adds the same partial sums up, and the results are the same bit for bit. */
 int candle_moe_router_topk(const void* hidden, const void* router_weight, void* topk_weight,
                            void* topk_indices, void* token_expert_indices, int num_tokens,
                            int hidden_dim, int num_experts, int topk, uint32_t dtype, void* stream);

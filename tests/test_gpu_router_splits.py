@@ -60,3 +60,33 @@ def test_capture(warm):
         assert np.array_equal(from_dev(out[1]).astype(np.uint32), wi)
         np.testing.assert_allclose(from_dev(out[0]), ww, rtol=1e-6, atol=0)
         run_fused(x, w, k, dt)  # the program's own work between replays
+
+
+@pytest.mark.parametrize("T,H,E,k,dt", [
+    (257, 2048, 128, 8, torch.bfloat16), (1000, 2056, 128, 8, torch.bfloat16),  # the exact and the f32 softmax
+    (2000, 2048, 128, 20, torch.float16), (700, 2880, 100, 4, torch.bfloat16),
+    (3283, 4096, 64, 8, torch.bfloat16), (1001, 4096, 40, 2, torch.float16),
+    (290, 1736, 65, 3, torch.float16),
+])
+def test_capture_gives_the_eager_bits(T, H, E, k, dt):
+    """Logits of every rounding: the captured call adds the K ranges up in the
+    order in which the eager one does and takes the same softmax."""
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(T + H)
+    x = torch.empty((T, H), dtype=dt, device="cuda").normal_(0.0, 1.0, generator=gen)
+    w = torch.empty((E, H), dtype=dt, device="cuda").normal_(0.0, 0.02, generator=gen)
+    eager, out = ([torch.zeros((T, k), dtype=d, device="cuda") for d in (torch.float32, torch.int32, torch.int32)]
+                  for _ in range(2))
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        candle_moe.router_topk(x, w, *out)
+    for _ in range(3):
+        for t in out:
+            t.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        candle_moe.router_topk(x, w, *eager)  # the program's own work between replays
+        for a, b in zip(eager, out):
+            assert torch.equal(a, b)
