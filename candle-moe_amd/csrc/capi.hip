@@ -23,6 +23,7 @@
 #include <stdarg.h>
 #include <stdio.h>
 
+#include <algorithm>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -130,7 +131,9 @@ int topk_softmax_impl(const void* g, int gdt, void* w, int wdt, void* idx, void*
 struct Problem {
     int T, H, I, E, k, act, moe_type, dtype;
     bool mfma;
-    bool f32_dec;  // f32 operands the decode kernels can load (16-byte chunks of 8 k)
+    bool f32_tiled;  // f32 operands the split-bf16 kernels can load (16-byte chunks of 4 k)
+    bool f32_dec;    // and the decode kernels (8 k)
+    bool fp8;
     bool packed;  // pre-packed K-contiguous 16-bit weights (candle_moe_fused_moe_packed)
     int cfg;  // TileCfg of both GEMMs
     int BM;
@@ -138,6 +141,7 @@ struct Problem {
     long long P;
     bool set_path;  // expert-set down projection (no atomics, no f32 accumulator)
     int nkeys;      // (E+1)^k expert-set keys
+    double set_from;  // nkeys > 0: tokens from which every prefill kernel's batches take the sets
     int split1;     // K splits of the gate/up GEMM (moe_lds_gemm only; > 1 needs partial + counters)
     int split2;     // K splits of the pair-path down GEMM (atomic combine)
     int n_tiles1, n_tiles2;
@@ -241,6 +245,8 @@ constexpr double kDecPartBytesF32 = 6.0 * 1024 * 1024;
 static size_t a256(size_t x) { return (x + 255) & ~(size_t)255; }
 size_t a256_bytes(size_t x) { return a256(x); }
 
+static size_t dec_part_bytes(const Problem& p);
+
 static Layout make_layout(const Problem& p) {
     Layout L;
     const size_t es = p.dtype == kF32 ? 4 : 2;
@@ -270,11 +276,7 @@ static Layout make_layout(const Problem& p) {
     L.inter = o; o += a256((size_t)p.P * p.I * es);
     L.acc = o;  // pair path: f32 accumulator [T, H], or the pair rows [T*k, H] (dtype)
     if (p.cfg == kDecGemv) {
-        // decode kernels: the f32 partials of both GEMMs (one after the other)
-        const size_t nc1 = (size_t)(p.moe_type == kQwen3 ? 2 : 1) * p.I;
-        const size_t n1 = p.dec_ks1 > 1 ? (size_t)p.dec_ks1 * p.P * nc1 : 0;  // (ks == 1: rows in the dtype)
-        const size_t n2 = (size_t)p.dec_ks2 * p.P * p.H;
-        o += a256(std::max(std::max(n1, n2) * 4, p.dtype == kF32 ? (size_t)kDecPartBytesF32 : 0));
+        o += a256(dec_part_bytes(p));  // decode kernels
     } else if (!p.set_path) {
         o += p.rows_path ? a256((size_t)p.P * p.H * es) : a256((size_t)p.T * p.H * 4);
     }
@@ -332,6 +334,46 @@ static int dec_slices(long long P, int N, int K, int kp, int nc_mult, double par
     ks = std::min<long long>(ks, kDecMaxSlices);
     ks = std::min<long long>(ks, (long long)(part_bytes / ((double)std::max<long long>(P, 1) * N * nc_mult * 4)));
     return (int)std::max<long long>(ks, 1);
+}
+// K slices of both decode GEMMs (p.cfg == kDecGemv) from the layer and the pairs.
+static void choose_dec_slices(Problem& p) {
+    const long long P = p.P;
+    p.dec_ks1 = p.dec_ks2 = 1;
+    // K slices for the gate/up (fc1) GEMM only where they paid: few
+    // column blocks of 128 and a large weight stream, or few and long
+    // blocks (below). Measured steps
+    // (router + forward, graph-replayed, cold bf16 weights), sliced
+    // against not: Qwen3 T=8 / 64 65.1 / 80.1 against 73.3 / 84.1 us;
+    // Qwen3-30B-A3B T=1 / 16 29.6 / 83.4 against 29.0 / 78.4 us, Nomic
+    // T=16 36.4 against 35.1 us (the finishing launch costs more than
+    // the faster stream saves); fp8 weights (half the bytes) slower
+    // sliced too. The down / fc2 GEMM, whose finishing launch sums the
+    // pairs anyway, ran 1-3 us faster unsliced on every shape.
+    const bool q3 = p.moe_type == kQwen3;
+    const long long groups = std::min<long long>(P, p.E);
+    const double wbytes = (double)groups * (q3 ? 2 : 1) * p.H * p.I * (p.fp8 ? 1 : p.dtype == kF32 ? 4 : 2);
+    // f32 (blocks of 64 columns): slices for the down / fc2 GEMM too where
+    // its items would leave CUs idle (Nomic's fc2 has 96 of them)
+    const int cols = p.dtype == kF32 ? 64 : 128;
+    const double part = p.dtype == kF32 ? kDecPartBytesF32 : kDecPartBytes;
+    // 16-bit also where the GEMM's 64-column blocks are few (a quarter of
+    // the CUs) and stream 1 MiB each: one or two tokens over large experts.
+    // Steps unsliced / sliced: Qwen3 T=1 36.0 / 27.8 us (pre-packed 38.0 /
+    // 34.3), H 8192 I 2048 k 1 T=1 85.6 / 37.9, H 4096 I 512 E 128 k 8 T=1
+    // 51.0 / 32.2. At 96 blocks (Qwen3 T=2) 57.9 / 43.0, but pre-packed,
+    // which takes the same slices to give the same bits, 48.2 / 51.1.
+    const bool few = p.dtype != kF32 && !p.fp8 && groups * cdiv(p.I, 64) <= 64 &&
+                     (long long)(q3 ? 2 : 1) * p.H * 128 >= (1 << 20);
+    if (groups * cdiv(p.I, cols) < 256 && (wbytes >= kDecSliceBytes || few))
+        p.dec_ks1 = dec_slices(P, p.I, p.H, q3 ? 2 : 4, q3 ? 2 : 1, part);
+    if (p.dtype == kF32 && groups * cdiv(p.H, cols) < 256) p.dec_ks2 = dec_slices(P, p.H, p.I, 4, 1, part);
+}
+// f32 partials of the decode GEMMs, one after the other in the same place.
+static size_t dec_part_bytes(const Problem& p) {
+    const size_t nc1 = (size_t)(p.moe_type == kQwen3 ? 2 : 1) * p.I;
+    const size_t n1 = p.dec_ks1 > 1 ? (size_t)p.dec_ks1 * p.P * nc1 : 0;  // (ks == 1: rows in the dtype)
+    const size_t n2 = (size_t)p.dec_ks2 * p.P * p.H;
+    return std::max(std::max(n1, n2) * 4, p.dtype == kF32 ? (size_t)kDecPartBytesF32 : 0);
 }
 // Workgroups of one round of the decode kernels: two per CU.
 static int dec_cap() { return 2 * 8 * std::max(cus_per_xcd(), 32); }
@@ -406,9 +448,10 @@ static int check_problem(int T, int H, int I, int E, int k, int act, uint32_t mo
     p.cfg = !p.mfma ? kTileSimt : (policy ? policy : kLds256w8);
     // f32: the split-bf16 kernels (decode kernels, 32-row or 128-row tiles)
     // wherever 16-byte loads are possible
-    const bool f32_tiled = p.dtype == kF32 && H % 4 == 0 && I % 4 == 0 && aligned16;
-    p.f32_dec = f32_dec && p.dtype == kF32 && H % 8 == 0 && I % 8 == 0 && aligned16;
-    if (f32_tiled) {
+    p.f32_tiled = p.dtype == kF32 && H % 4 == 0 && I % 4 == 0 && aligned16;
+    p.f32_dec = f32_dec && p.f32_tiled && H % 8 == 0 && I % 8 == 0;
+    p.fp8 = fp8;
+    if (p.f32_tiled) {
         // 32-row tiles up to 64 rows per touched expert (steps, 32-row against
         // 128-row tiles: Nomic T=129 / 256 118 / 109 against 141 / 153 us,
         // Qwen3 T=140 / 200 239 / 220 against 306 / 309 us; beyond, Qwen3
@@ -513,6 +556,7 @@ static int check_problem(int T, int H, int I, int E, int k, int act, uint32_t mo
     // 404 us at T=12288).
     p.set_path = false;
     p.nkeys = 0;
+    p.set_from = 0.0;
     // (fp8 weights: on the 8-wave prefill kernel, whose expert-set GEMM keeps
     // its accumulators in per-segment column units)
     if (p.mfma && (!fp8 || p.cfg == kLds256w8) && out16 && (I % 64) == 0 && k <= kSetMaxK &&
@@ -532,6 +576,7 @@ static int check_problem(int T, int H, int I, int E, int k, int act, uint32_t mo
             // Nomic T=12288 / 32768 pairs 377 / 859 against 390 / 899 us.
             const bool rows_ok = p.mfma && is_lds_cfg(p.cfg) && p.dtype != kF32;
             const bool big_rows = (double)P * H * 2.0 >= (double)kSetMinRowBytes;
+            p.set_from = std::max(fill * 256 * sets, kSetMinRowBytes / (2.0 * H * k));
             p.set_path = p.cfg != kDecGemv &&
                          (g_combine_policy == 2 ||
                           (p.cfg != kLdsRows32 && (double)T >= fill * p.BM * sets && (!rows_ok || big_rows)));
@@ -625,58 +670,82 @@ static int check_problem(int T, int H, int I, int E, int k, int act, uint32_t mo
         p.split1 = choose(mt * p.n_tiles1, H);
     }
     p.dec_ks1 = p.dec_ks2 = 1;
-    if (p.cfg == kDecGemv) {
-        // K slices for the gate/up (fc1) GEMM only where they paid: few
-        // column blocks of 128 and a large weight stream, or few and long
-        // blocks (below). Measured steps
-        // (router + forward, graph-replayed, cold bf16 weights), sliced
-        // against not: Qwen3 T=8 / 64 65.1 / 80.1 against 73.3 / 84.1 us;
-        // Qwen3-30B-A3B T=1 / 16 29.6 / 83.4 against 29.0 / 78.4 us, Nomic
-        // T=16 36.4 against 35.1 us (the finishing launch costs more than
-        // the faster stream saves); fp8 weights (half the bytes) slower
-        // sliced too. The down / fc2 GEMM, whose finishing launch sums the
-        // pairs anyway, ran 1-3 us faster unsliced on every shape.
-        const bool q3 = p.moe_type == kQwen3;
-        const long long groups = std::min<long long>(P, E);
-        const double wbytes = (double)groups * (q3 ? 2 : 1) * H * I * (fp8 ? 1 : p.dtype == kF32 ? 4 : 2);
-        // f32 (blocks of 64 columns): slices for the down / fc2 GEMM too where
-        // its items would leave CUs idle (Nomic's fc2 has 96 of them)
-        const int cols = p.dtype == kF32 ? 64 : 128;
-        const double part = p.dtype == kF32 ? kDecPartBytesF32 : kDecPartBytes;
-        // 16-bit also where the GEMM's 64-column blocks are few (a quarter of
-        // the CUs) and stream 1 MiB each: one or two tokens over large experts.
-        // Steps unsliced / sliced: Qwen3 T=1 36.0 / 27.8 us (pre-packed 38.0 /
-        // 34.3), H 8192 I 2048 k 1 T=1 85.6 / 37.9, H 4096 I 512 E 128 k 8 T=1
-        // 51.0 / 32.2. At 96 blocks (Qwen3 T=2) 57.9 / 43.0, but pre-packed,
-        // which takes the same slices to give the same bits, 48.2 / 51.1.
-        const bool few = p.dtype != kF32 && !fp8 && groups * cdiv(I, 64) <= 64 &&
-                         (long long)(q3 ? 2 : 1) * H * 128 >= (1 << 20);
-        if (groups * cdiv(I, cols) < 256 && (wbytes >= kDecSliceBytes || few))
-            p.dec_ks1 = dec_slices(P, I, H, q3 ? 2 : 4, q3 ? 2 : 1, part);
-        if (p.dtype == kF32 && groups * cdiv(H, cols) < 256) p.dec_ks2 = dec_slices(P, H, I, 4, 1, part);
-    }
+    if (p.cfg == kDecGemv) choose_dec_slices(p);
     return CANDLE_MOE_OK;
 }
 
-// Most workspace a smaller batch of the same layer (dtype, sizes, combine
-// policy) needs: the kernels that take smaller batches keep more of it in
-// places (decode partials by slice, K-split partials). A workspace allocated,
-// or sized by the caller, for a batch has to do for the smaller ones too, also
-// under graph capture, where it cannot grow. Asked at the largest batch of
-// each kernel's range.
-static size_t smaller_batches_ws(const Problem& p, bool fp8) {
-    const long long P_at[] = {kDecDefaultPairs, 32LL * p.E, 64LL * p.E, 128LL * p.E, kOneTileRows * p.E, 256LL * p.E - 1};
-    size_t most = 0;
-    for (long long P : P_at) {
-        const long long T = P / p.k;
-        Problem q;
-        if (T < 1 || T >= p.T ||
-            check_problem((int)T, p.H, p.I, p.E, p.k, p.act, (uint32_t)p.moe_type, (uint32_t)p.dtype, q, true, true, fp8,
-                          p.packed))
-            continue;
-        most = std::max(most, make_layout(q).total);
+// Workspace bytes that serve every batch of 1 .. p.T tokens of p's layer
+// (dtype, sizes, policies), at least make_layout(p).total. The need of a batch
+// does not grow with it: decode partials by slice, K-split partials, the pairs'
+// rows and the f32 accumulator come and go with the kernels, their split counts
+// and the expert sets. A workspace for a batch, the caller's or the library's,
+// has to do for the smaller ones, in a captured call too, where it cannot grow.
+// So each part is taken at its most over all kernels within reach of 1 .. p.T
+// tokens; every part below grows with p.T, hence so does the sum.
+static size_t upto_bytes(const Problem& p) {
+    const size_t exact = make_layout(p).total;
+    if (!p.mfma && !p.f32_tiled) return exact;  // one kernel for every batch
+    const long long P = p.P, E = p.E, touched = std::min(P, E);
+    const bool f32 = p.dtype == kF32, forced = g_tile_policy != 0;
+    const size_t es = f32 ? 4 : 2;
+    const long long tiles = grouping_max_tiles(P, p.E, 32);  // (the lowest row tile)
+    size_t o = kWsHeaderBytes + a256((size_t)(E + 2) * 4) + a256((size_t)std::max<long long>(grouping_blocks(P), 1) * E * 4) +
+               a256((size_t)P * 4) + 2 * a256((size_t)tiles * 4) + 256 + a256((size_t)P * p.I * es) + 256;
+    if (p.nkeys > 0 && (P > 32 * touched || g_combine_policy == 2)) {
+        const size_t sets = (size_t)((p.T + 31) / 32 + std::min<long long>(p.nkeys, p.T));
+        o += a256((size_t)(p.nkeys + 2) * 4) + a256((size_t)std::max<long long>(grouping_blocks(p.T), 1) * p.nkeys * 4) +
+             a256((size_t)p.T * 4) + 2 * a256(sets * 4) + 256 + a256((size_t)P * 4);
     }
-    return most;
+
+    size_t acc = 0, partial = 0;
+    // decode kernels: the partials of both GEMMs by slices
+    const bool any_rows = p.fp8 || g_tile_policy == kDecGemv;  // (else up to 32 rows per touched expert)
+    const long long most = g_tile_policy == kDecGemv ? kDecMaxPairs : p.fp8 ? kW8DecPairs : kDecDefaultPairs;
+    const long long dec_pairs = any_rows ? most : std::min(most, 32 * E);
+    Problem q = p;
+    q.cfg = kDecGemv;
+    bool dec = dec_pairs >= p.k;
+    for (long long t = 1; dec && t <= p.T && t * p.k <= dec_pairs; ++t) {
+        q.T = (int)t;
+        q.P = t * p.k;
+        dec = dec_gemv_fits(q);
+        choose_dec_slices(q);
+        acc = std::max(acc, dec_part_bytes(q));
+    }
+    if (!dec || forced || P > dec_pairs) {
+        const int n1 = cdiv(p.I, 64), n2 = cdiv(p.H, 64);  // (the narrowest column tile)
+        o += a256((size_t)tiles * std::max(n1, n2) * 4);   // split-K counters
+        if (f32) {
+            acc = std::max(acc, (size_t)p.T * p.H * 4);
+            // K splits of the tile kernels, at most 16, where the expected tiles
+            // number less than 256: up to ceil(512 / tiles). The slots cover the
+            // most tiles there can be, at most twice the expected ones, of each.
+            auto splits = [&](int bm, long long pairs) {
+                const long long est = std::max((pairs + bm - 1) / bm, std::min(pairs, E)) * std::max(n1, n2);
+                return (size_t)std::min(2 * (512 + 255LL), 2 * 16 * est) * bm * 128 * 4;
+            };
+            partial = splits(32, forced ? P : std::min(P, 64 * E));
+            if (forced || P > 64 * touched) partial = std::max(partial, splits(128, P));
+        } else {
+            // 32-row kernels: f32 atomics, one round of K splits
+            const long long rows32 = forced ? P : std::min(P, (p.fp8 ? 256 : 128) * E);
+            acc = std::max(acc, (size_t)(rows32 / p.k) * p.H * 4);
+            partial = (size_t)(cus_per_xcd() > 0 ? 8 * cus_per_xcd() : 256) * 32 * tile_cols(kLdsRows32) * 4;
+            // the others: the pairs' rows until the expert sets take over; the
+            // 256x256 kernel's K-split tail
+            if (forced || P > 32 * touched) {
+                double t = p.T;
+                if (p.set_path && g_combine_policy == 0) t = std::min(t, std::ceil(p.set_from));
+                acc = std::max(acc, (size_t)std::min(t * p.k * p.H * 2.0, kRowsMaxBytes));
+            }
+            if (forced || P > (p.fp8 ? 32 : kOneTileRows) * touched) {
+                const size_t slots = 8 * (size_t)cus_per_xcd();
+                partial = std::max(partial, slots * 256 * tile_cols(kLds256w8) * 4);
+                o += a256(slots * 4);
+            }
+        }
+    }
+    return std::max(exact, o + a256(acc) + a256(partial));
 }
 
 // fp8 expert weights of candle_moe_fused_moe_fp8 (codes [E][N][K], scales [E][N])
@@ -1053,6 +1122,13 @@ struct OwnedWs {
     size_t bytes;
     bool captured;  // a graph may hold ptr
     std::vector<void*> replaced;
+    // layers (and the policies then) that it serves up to a number of tokens,
+    // so that upto_bytes is not worked out again in every call
+    struct Served {
+        long long layer[8];
+        int T;
+    } served[4];
+    unsigned next;
 };
 static std::mutex g_ws_mu;
 static std::vector<OwnedWs> g_ws;
@@ -1061,21 +1137,24 @@ static std::vector<OwnedWs> g_ws;
 // (err = hipErrorStreamCaptureUnsupported): hipMallocAsync there would add an
 // allocation node to the caller's graph, memory the graph owns and releases
 // when it is destroyed, while this table would keep handing it out.
-// reserve: bytes to allocate at least, asked for when the workspace grows.
 static bool is_capturing(hipStream_t s) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &cs) == hipSuccess) return cs != hipStreamCaptureStatusNone;
     (void)hipGetLastError();
     return false;
 }
-template <class F>
-static OwnedWs* owned_ws_locked(int dev, hipStream_t s, size_t need, hipError_t& err, F&& reserve) {
-    err = hipSuccess;
-    OwnedWs* w = nullptr;
+// A captured call takes what holds its need; others have the workspace grown to
+// `reserve` (>= need) bytes first, if there is memory for it.
+static OwnedWs* find_ws_locked(int dev, hipStream_t s) {
     for (auto& e : g_ws)
-        if (e.device == dev && e.stream == s) w = &e;
+        if (e.device == dev && e.stream == s) return &e;
+    return nullptr;
+}
+static OwnedWs* owned_ws_locked(int dev, hipStream_t s, size_t need, size_t reserve, hipError_t& err) {
+    err = hipSuccess;
+    OwnedWs* w = find_ws_locked(dev, s);
     const bool capturing = is_capturing(s);
-    if (w && w->bytes >= need) {
+    if (w && w->bytes >= (capturing ? need : reserve)) {
         w->captured = w->captured || capturing;
         return w;
     }
@@ -1085,10 +1164,20 @@ static OwnedWs* owned_ws_locked(int dev, hipStream_t s, size_t need, hipError_t&
     }
     // grow by at least 1.5x and to whole MiB, so that a slowly growing T
     // does not reallocate on every call
-    size_t want = std::max(need + need / 2, (size_t)reserve());
+    size_t want = std::max(reserve, need + need / 2);
+    if (w) want = std::max(want, w->bytes + w->bytes / 2);
     want = (want + (1u << 20) - 1) & ~(size_t)((1u << 20) - 1);
     void* mem = nullptr;
     err = hipMallocAsync(&mem, want, s);
+    if (err != hipSuccess) {
+        (void)hipGetLastError();
+        if (w && w->bytes >= need) {
+            err = hipSuccess;
+            return w;
+        }
+        want = need;
+        err = hipMallocAsync(&mem, want, s);
+    }
     if (err != hipSuccess) return nullptr;
     // the header's counters start at zero (a kernel, not a memset node,
     // should the call be captured into a graph)
@@ -1105,7 +1194,7 @@ static OwnedWs* owned_ws_locked(int dev, hipStream_t s, size_t need, hipError_t&
         w->captured = false;
         return w;
     }
-    g_ws.push_back(OwnedWs{dev, s, mem, want, false, {}});
+    g_ws.push_back(OwnedWs{dev, s, mem, want, false, {}, {}, 0});
     return &g_ws.back();
 }
 
@@ -1167,9 +1256,21 @@ int fused_moe_impl(const void* x, const void* gate, const void* up, const void* 
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return hip_fail(e, "fused_moe: hipGetDevice");
     std::lock_guard<std::mutex> lk(g_ws_mu);
-    // (asked for only where the workspace has to grow)
-    const auto reserve = [&]() { return aligned16 ? smaller_batches_ws(p, f8 != nullptr) : (size_t)0; };
-    OwnedWs* w = owned_ws_locked(dev, s, L.total, e, reserve);
+    OwnedWs* w = find_ws_locked(dev, s);
+    const long long layer[8] = {p.H, p.I, p.E, p.k, p.dtype | p.moe_type << 4 | (int)p.fp8 << 5 | (int)p.packed << 6,
+                                (int)aligned16 | (int)p.set_path << 1, g_tile_policy, g_combine_policy};
+    int slot = -1;
+    if (w)
+        for (int i = 0; i < 4; ++i)
+            if (std::equal(layer, layer + 8, w->served[i].layer)) slot = i;
+    const bool served = slot >= 0 && T <= w->served[slot].T;
+    const size_t full = served ? L.total : upto_bytes(p);
+    w = owned_ws_locked(dev, s, L.total, full, e);
+    if (w && !served && w->bytes >= full) {
+        if (slot < 0) slot = w->next++ & 3;
+        std::copy(layer, layer + 8, w->served[slot].layer);
+        w->served[slot].T = T;
+    }
     if (!w) return ws_fail("fused_moe", L.total, e);
     return run_moe(p, x, gate, up, down, reinterpret_cast<const float*>(rw), reinterpret_cast<const uint32_t*>(idx),
                    out, overwrite, reinterpret_cast<char*>(w->ptr), s, f8, true);
@@ -1253,7 +1354,7 @@ size_t fused_moe_ws_size(int T, int H, int I, int E, int k, uint32_t dtype) {
         for (int al = 0; al < 2; ++al) {
             Problem p;
             if (check_problem(T, H, I, E, k, 0, mt, dtype, p, al != 0)) return 0;
-            most = std::max(most, std::max(make_layout(p).total, al ? smaller_batches_ws(p, false) : (size_t)0));
+            most = std::max(most, upto_bytes(p));
         }
     return most;
 }
@@ -1452,18 +1553,20 @@ int candle_moe_router_topk(const void* hidden, const void* router_weight, void* 
     // (after the workspace header, whose counters stay zero)
     // A captured call of more than kRouterSplitTokens tokens needs no workspace
     // (its stream may have none): the same sums in one pass.
-    const bool one_pass =
-        T > cm::kRouterSplitTokens && cm::router_splits(T, H, E, (int)dtype) > 1 && cm::is_capturing(s);
-    const size_t rneed = one_pass ? 0 : cm::router_ws_bytes(T, H, E, (int)dtype);
-    const size_t need = rneed > 0 ? cm::kWsHeaderBytes + rneed : 0;
+    // (And a larger call that runs in one pass anyway still sees to the workspace
+    // of the smaller ones captured after it.)
+    const bool large = T > cm::kRouterSplitTokens;
+    const size_t rupto = cm::router_upto_bytes(T, H, E, (int)dtype);
+    const size_t rneed = large && rupto > 0 && cm::is_capturing(s) ? 0 : rupto;
     hipError_t e = hipSuccess;
-    if (need > 0) {
+    if (rneed > 0) {
+        const size_t need = cm::kWsHeaderBytes + cm::router_ws_bytes(T, H, E, (int)dtype);
         int dev = 0;
         e = hipGetDevice(&dev);
         if (e != hipSuccess) return cm::hip_fail(e, "router_topk: hipGetDevice");
         std::lock_guard<std::mutex> lk(cm::g_ws_mu);
-        cm::OwnedWs* w = cm::owned_ws_locked(dev, s, need, e, [] { return (size_t)0; });
-        if (!w && T <= cm::kRouterSplitTokens) return cm::ws_fail("router_topk", need, e);
+        cm::OwnedWs* w = cm::owned_ws_locked(dev, s, need, cm::kWsHeaderBytes + rneed, e);
+        if (!w && !large) return cm::ws_fail("router_topk", need, e);
         if (!w) (void)hipGetLastError();  // (no memory for it: one pass)
         e = cm::launch_router_topk(hidden, router_weight, (int)dtype, reinterpret_cast<float*>(topk_weight),
                                    reinterpret_cast<uint32_t*>(topk_indices),

@@ -15,10 +15,13 @@ hipError_t launch_router_topk(const void* x, const void* w, int dtype, float* wo
                               int H, int E, int k, hipStream_t stream, float* part = nullptr,
                               size_t part_bytes = 0);
 // Up to kRouterSplitTokens tokens the K split needs its workspace (as it always
-// did); larger batches run in one pass under graph capture and where there is none.
+// did); larger batches do without under graph capture and where there is none.
 constexpr int kRouterSplitTokens = 256;
 int router_splits(int T, int H, int E, int dtype);
 size_t router_ws_bytes(int T, int H, int E, int dtype);
+// Bytes for T tokens and for every smaller batch that needs the workspace while
+// captured: fewer tokens can take more splits.
+size_t router_upto_bytes(int T, int H, int E, int dtype);
 hipError_t launch_topk_softmax(const void* logits, int in_dtype, void* w, int w_dtype, uint32_t* idx,
                                uint32_t* ei, int T, int E, int k, hipStream_t stream);
 // test support: the router's f32 exponential against its f64 one

@@ -1238,6 +1238,12 @@ size_t router_ws_bytes(int T, int H, int E, int dtype) {
     const int ks = router_splits(T, H, E, dtype);
     return ks > 1 ? (size_t)ks * T * E * sizeof(float) : 0;
 }
+size_t router_upto_bytes(int T, int H, int E, int dtype) {
+    size_t most = router_ws_bytes(T, H, E, dtype);
+    for (int t = 32; t < T + 32 && t <= kRouterSplitTokens; t += 32)  // (the most tokens of each tile count)
+        most = std::max(most, router_ws_bytes(std::min(t, T), H, E, dtype));
+    return most;
+}
 
 template <int DT, int NB>
 static hipError_t launch_router_split(const void* x, const void* w, float* wo, uint32_t* io, uint32_t* eo, int T,

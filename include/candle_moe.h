@@ -79,7 +79,8 @@ void topk_softmax(const void* gating_output, void* topk_weight, void* topk_indic
  * being captured into a graph gets no new or larger workspace (the graph
  * would own that memory): such a call fails with CANDLE_MOE_ERR_WORKSPACE
  * before enqueuing anything, so make one call of the largest size on the
- * stream before capturing it.
+ * stream before capturing it: the workspace then holds every smaller batch of
+ * that layer, whichever kernels it takes.
  */
 void fused_moe(const void* input, const void* gate_weights, const void* up_weights,
                const void* down_weights, const void* routing_weights, const void* expert_indices,
@@ -110,8 +111,8 @@ int candle_moe_fused_moe_status(const void* input, const void* gate_weights, con
                                 uint32_t dtype, void* stream);
 
 /* Caller-provided workspace: bytes needed by candle_moe_fused_moe_ws for
- * these sizes, for either moe_type and any operand alignment (0 when the
- * arguments are invalid). */
+ * these sizes and for every smaller num_tokens, for either moe_type and any
+ * operand alignment (0 when the arguments are invalid). */
 size_t candle_moe_fused_moe_workspace_size(int num_tokens, int hidden_dim, int intermediate_dim,
                                            int num_experts, int num_selected_experts,
                                            uint32_t dtype);

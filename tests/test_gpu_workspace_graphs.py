@@ -114,3 +114,71 @@ def test_layer_graph_outlives_a_larger_call():
     del g
     candle_moe.trim_workspaces()
     assert pool_bytes() == empty
+
+
+def forward_case(T, H, I, E, k, dt):
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(T)
+    x, G, U, D = (torch.empty(s, dtype=dt, device="cuda").normal_(0.0, d, generator=gen)
+                  for s, d in (((T, H), 1.0), ((E, H, I), 0.02), ((E, H, I), 0.02), ((E, I, H), 0.02)))
+    idx = torch.rand((T, E), device="cuda", generator=gen).argsort(1)[:, :k].to(torch.int32).contiguous()
+    return x, G, U, D, torch.full((T, k), 1.0 / k, device="cuda"), idx
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("H,I,E,k,most,fewer", [(2048, 768, 128, 8, 6, (1, 5)), (4096, 512, 8, 2, 2, (1,)),
+                                                (1280, 1888, 64, 2, 120, (3, 17, 64, 99)),
+                                                (768, 3072, 8, 2, 300, (128, 129, 200))])
+@pytest.mark.parametrize("pregrown", [False, True])
+def test_one_call_of_the_largest_size(H, I, E, k, most, fewer, dt, pregrown):
+    """After one eager call the smaller batches of the layer can be captured,
+    also where another call's workspace was there and held that eager call."""
+    candle_moe.trim_workspaces()
+    s = torch.cuda.Stream()
+    moe = candle_moe.FusedMoE.new(E, k, candle_moe.Activation.Silu)
+    x, G, U, D, w, idx = forward_case(most, H, I, E, k, dt)
+    xr, wr, _ = router_case(1000, 2048, 128, 8, O.BF16)
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        if pregrown:
+            candle_moe.router_topk(xr, wr, *outputs(1000, 8))
+        moe.forward(x, G, U, D, w, idx, 0)
+    torch.cuda.synchronize()
+    for T in fewer:
+        args = x[:T].contiguous(), G, U, D, w[:T].contiguous(), idx[:T].contiguous(), 0
+        want = moe.forward(*args)
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            out = moe.forward(*args)
+        for _ in range(2):
+            out.zero_()
+            g.replay()
+            torch.cuda.synchronize()
+            # (K splits of few tiles meet in f32 atomics: the last bits may differ)
+            assert (out - want).norm() <= (1e-2 if dt is torch.bfloat16 else 1e-5) * want.norm(), T
+        del g
+
+
+@pytest.mark.parametrize("most,fewer", [(129, 128), (4099, 200), (1000, 256)])
+def test_router_after_a_larger_call(most, fewer):
+    H, E, k, dt = 2048, 128, 8, O.BF16
+    candle_moe.trim_workspaces()
+    s = torch.cuda.Stream()
+    xl, wl, _ = router_case(most, H, E, k, dt)
+    x, w, (ww, wi, _) = router_case(fewer, H, E, k, dt)
+    small = forward_case(1, 256, 128, 4, 2, torch.bfloat16)
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):  # (the layer's workspace of 1 MiB is there first)
+        candle_moe.FusedMoE.new(4, 2, candle_moe.Activation.Silu).forward(*small, 0)
+        candle_moe.router_topk(xl, wl, *outputs(most, k))
+    torch.cuda.synchronize()
+    out = outputs(fewer, k)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        candle_moe.router_topk(x, w, *out)
+    for _ in range(2):
+        g.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(from_dev(out[1]).astype(np.uint32), wi)
+        np.testing.assert_allclose(from_dev(out[0]), ww, rtol=1e-6, atol=0)

@@ -36,9 +36,26 @@ def test_kernel_at_the_lines(H, I, E, k, rows, code):
 @pytest.mark.parametrize("H,I,E,k", [(4096, 1536, 8, 2), (2048, 768, 128, 8), (768, 3072, 8, 2), (1024, 2048, 16, 2),
                                      (520, 264, 5, 3)])
 def test_workspace_past_a_line(H, I, E, k, dt):
-    """Past a line the workspace still holds the largest batch before it."""
+    """Past a line the workspace still holds the largest batch before it. (The
+    lines that lie at a number of rows; the next test has all batches.)"""
     size = cm.lib().candle_moe_fused_moe_workspace_size
     lines = sorted({256 // k} | {r * E // k for r in (32, 64, 128, 136)} | {(256 * E - 1) // k})
     for i, T in enumerate(lines):
         for larger in [T + 1] + lines[i + 1:] + [2 * lines[-1]]:
             assert size(larger, H, I, E, k, dt) >= size(T, H, I, E, k, dt) > 0, (T, larger)
+
+
+@pytest.mark.parametrize("dt", [cm.DT_BF16, cm.DT_F16, cm.DT_F32])
+@pytest.mark.parametrize("H,I,E,k", [(4096, 1536, 8, 2), (2048, 768, 128, 8), (768, 3072, 8, 2), (4096, 4096, 128, 1),
+                                     (1280, 1888, 64, 2), (8192, 2048, 8, 1), (4096, 512, 128, 8), (520, 264, 5, 3),
+                                     (1536, 2048, 256, 4), (4096, 4096, 1, 1), (516, 260, 6, 2), (257, 129, 4, 2)])
+def test_workspace_never_shrinks(H, I, E, k, dt):
+    """A workspace for a batch does for every smaller one: its size never falls
+    from one number of tokens to the next (decode slices, K splits, the pairs'
+    rows and the expert sets all come and go on the way)."""
+    size = cm.lib().candle_moe_fused_moe_workspace_size
+    last = 0
+    for T in list(range(1, 1200)) + list(range(1200, 6000, 7)) + list(range(6000, 40000, 211)):
+        n = size(T, H, I, E, k, dt)
+        assert n >= last > 0 or (T == 1 and n > 0), (T, last, n)
+        last = n
