@@ -3,9 +3,9 @@
 // gfx950 has no f32 matrix rate above its vector FMA rate (157 TFLOP/s
 // nominal; the vector form of this kernel reached 62 TFLOP/s at Nomic
 // T=4096), while a bf16 MFMA runs 16 times that rate. Every f32 value is
-// therefore split into three bf16 parts, x = h + m + l: h = bf16(x), m =
-// bf16(x - h), l = bf16(x - h - m), all rounded to nearest even, the
-// differences exact, so that the parts hold all 24 significand bits. A
+// therefore split into three bf16 parts, 2^16 x = h + m + l: h = bf16(2^16 x),
+// m and l likewise of what is left, all rounded to nearest even, the
+// differences exact, so that the parts hold all 24 significand bits (split2). A
 // product is summed from the six part products of relative size 2^-18 and
 // above (l*h, h*l, m*m, m*h, h*m, h*h, smallest first), accumulated in f32 by
 // the MFMA; the dropped ones (m*l, l*m, l*l) are below 2^-26 of it, a quarter
@@ -21,9 +21,9 @@
 // Bound: the matrix cores at the clock the chip holds under them (without the
 // loads and the splits the same loop takes 214 us for that fc1).
 //
-// Values the split cannot hold (infinities, NaN, magnitudes that round to a
-// bf16 infinity) give a non-finite sum in every output they enter; such
-// blocks (and sums that overflow f32) are recomputed with plain f32 FMAs
+// Values the split cannot hold (infinities, NaN, magnitudes from 2^111) give a
+// non-finite sum in every output they enter; such
+// blocks (and sums from 2^96, which overflow scaled) are recomputed with plain f32 FMAs
 // from the operands in memory, so non-finite inputs give what the vector
 // kernel gave.
 //
@@ -286,7 +286,7 @@ __global__ __launch_bounds__(256, 2) void moe_f32_gemm(GemmArgs a) {
 #pragma unroll
         for (int j = 0; j < NB; ++j)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] += small[i][j][r];
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = (acc[i][j][r] + small[i][j][r]) * kSplitUnscale;
 
     // Blocks with a non-finite sum again with f32 FMAs (see the top). Register
     // i of lane l: row 8(i/4) + 4(l/32) + i%4 of the block, column l%32.

@@ -591,9 +591,10 @@ __global__ __launch_bounds__(64 * kDvWaves, 2) void moe_dec_gemv(DecArgs a) {
 #pragma unroll
                 for (int b = 0; b < NB; ++b)
 #pragma unroll
-                    for (int v = 0; v < 4; ++v) acc[rb][b][v] += small[rb][b][v];
-            // blocks with a non-finite sum (infinities, NaN, values whose bf16
-            // part rounds to infinity, overflow) again with f32 FMAs over this
+                    for (int v = 0; v < 4; ++v)
+                        acc[rb][b][v] = (acc[rb][b][v] + small[rb][b][v]) * kSplitUnscale;
+            // blocks with a non-finite sum (infinities, NaN, values whose scaled
+            // bf16 part rounds to infinity, overflow) again with f32 FMAs over this
             // wave's k (an element past the operands reads zero)
 #pragma unroll
             for (int b = 0; b < NB; ++b) {

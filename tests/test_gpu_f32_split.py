@@ -80,3 +80,24 @@ def test_f32_split_non_finite_and_extreme_inputs(tile, mt):
             assert np.isfinite(w).all() == np.isfinite(g).all(), t
             if np.isfinite(w).all():
                 assert np.linalg.norm(g - w) <= 1e-5 * np.linalg.norm(w) + 1e-44, t
+
+
+@pytest.mark.parametrize("tile", [0, 15, 16])
+@pytest.mark.parametrize("mt,tiny", [(O.NOMIC, "x"), (O.NOMIC, "gate"), (O.NOMIC, "up"), (O.QWEN3, "gate"), (O.QWEN3, "down")])
+@pytest.mark.parametrize("scale", [1e-36, 1e-38, 1e-41])
+def test_f32_split_tiny_operands(tile, mt, tiny, scale):
+    """One operand tiny, subnormal ones included, the others such that every sum
+    stays in f32's normal range: the parts still hold every bit, so the bound is
+    that of ordinary values. (Unscaled parts lost the bits below 2^-133: 2.6e-5
+    at 1e-36, 2.6e-3 at 1e-38.)"""
+    T, H, I, E, k = 40, 256, 192, 2, 1
+    x, G, U, D, rw, ri = moe_inputs(T, H, I, E, k, O.F32, 970, mt, wstd=1.0)
+    ops = {"x": x, "gate": G, "up": U, "down": D}
+    for name, t in ops.items():
+        if t is not None:
+            t *= np.float32(scale if name == tiny else 100.0)
+    G *= np.float32(100.0 if tiny != "gate" else 1.0)
+    got = _forward(x, G, U, D, rw, ri, E, k, O.RELU, mt, tile).astype(np.float64)
+    want = O.fused_moe(x, G, U, D, rw, ri, E=E, k=k, act=O.RELU, moe_type=mt, dtype=O.F32, mode=O.MODE_EXACT)
+    err = np.linalg.norm(got / scale - want / scale) / np.linalg.norm(want / scale)
+    assert err <= REL, err
