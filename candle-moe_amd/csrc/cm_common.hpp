@@ -87,6 +87,50 @@ __device__ __forceinline__ void split8(const float (&v)[8], u32x4& h, u32x4& m, 
     }
 }
 
+// Non-finite sums of a split-bf16 block (infinities, NaN and values or sums beyond
+// the split's range) again with f32 FMAs over k0 .. k1 - 1 (multiples of 4). A wave
+// holds R registers of sums; the lanes of a group of GL share the row of
+// register q. get / set: this lane's sum q; a4(q, k): four operands of its row;
+// b(k): its column's. A row with a NaN has NaN in all its sums already: its GL
+// lanes look for one first, and a row of padding ends there (with all sums of the
+// block recomputed, one NaN row made a call 7 to 15 times as long).
+template <int R, int GL, class Get, class Set, class A4, class B>
+__device__ __forceinline__ void redo_non_finite(int lane, int k0, int k1, Get get, Set set, A4 a4, B b) {
+    const uint64_t group = (GL == 32 ? 0xffffffffull : 0xffffull) << (lane & (64 - GL));
+#pragma unroll 1
+    for (int q = 0; q < R; ++q) {
+        const bool bad = !__builtin_isfinite(get(q));
+        bool todo = bad, nan = false;
+        for (int kb = k0; kb < k1 && __any(todo); kb += 4 * GL) {
+            const int k = kb + 4 * (lane % GL);
+            if (k < k1) {
+                const f32x4 v = a4(q, k);
+                nan = nan || v[0] != v[0] || v[1] != v[1] || v[2] != v[2] || v[3] != v[3];
+            }
+            todo = bad && (__builtin_amdgcn_ballot_w64(nan) & group) == 0ull;
+        }
+        float s = 0.f;
+        int k = k0;
+        // (NaN stays: a row of infinities ends at the first change of sign)
+        for (; k + 16 <= k1 && __any(todo && s == s); k += 16) {
+            f32x4 x[4];
+            float w[16];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) x[i] = a4(q, k + 4 * i);
+#pragma unroll
+            for (int i = 0; i < 16; ++i) w[i] = b(k + i);
+#pragma unroll
+            for (int i = 0; i < 16; ++i) s = fmaf(x[i / 4][i % 4], w[i], s);
+        }
+        for (; k < k1 && __any(todo && s == s); k += 4) {
+            const f32x4 x = a4(q, k);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) s = fmaf(x[i], b(k + i), s);
+        }
+        if (todo) set(q, s);
+    }
+}
+
 template <int DT> struct Elem;
 template <> struct Elem<kBF16> {
     typedef uint16_t storage;

@@ -593,9 +593,8 @@ __global__ __launch_bounds__(64 * kDvWaves, 2) void moe_dec_gemv(DecArgs a) {
 #pragma unroll
                     for (int v = 0; v < 4; ++v)
                         acc[rb][b][v] = (acc[rb][b][v] + small[rb][b][v]) * kSplitUnscale;
-            // blocks with a non-finite sum (infinities, NaN, values whose scaled
-            // bf16 part rounds to infinity, overflow) again with f32 FMAs over this
-            // wave's k (an element past the operands reads zero)
+            // non-finite sums (infinities, NaN, values whose scaled bf16 part
+            // rounds to infinity, overflow) again with f32 FMAs over this wave's k
 #pragma unroll
             for (int b = 0; b < NB; ++b) {
                 bool bad = false;
@@ -604,31 +603,31 @@ __global__ __launch_bounds__(64 * kDvWaves, 2) void moe_dec_gemv(DecArgs a) {
 #pragma unroll
                     for (int v = 0; v < 4; ++v) bad |= !__builtin_isfinite(acc[rb][b][v]);
                 if (__builtin_expect(__any(bad), 0)) {
-                    uint32_t arow[RB][4];
-#pragma unroll
-                    for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-                        for (int v = 0; v < 4; ++v) {
-                            const int m = rb * 16 + 4 * g + v;
-                            const int p = s_rows[c0 + min(m, m_valid - 1)];
-                            arow[rb][v] = (uint32_t)(GATHER ? p / a.k_top : p) * (uint32_t)K * 4u;
-                            acc[rb][b][v] = 0.f;
-                        }
                     const int col = min(ncol[b], N - 1);
-                    const int k_hi = min(K, s_hi * KSTEP);
-                    for (int k = s_lo * KSTEP; k < k_hi; ++k) {
-                        const uint32_t wo = TRANS ? (uint32_t)k * ldb2 + 4u * (uint32_t)col
-                                                  : (uint32_t)col * ldb2 + 4u * (uint32_t)k;
-                        const float w = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rw, wo, 0, 0));
+                    redo_non_finite<4 * RB, 16>(
+                        lane, s_lo * KSTEP, min(K, s_hi * KSTEP),
+                        [&](int q) {
+                            float r = 0.f;
 #pragma unroll
-                        for (int rb = 0; rb < RB; ++rb)
+                            for (int i = 0; i < 4 * RB; ++i) r = q == i ? acc[i / 4][b][i % 4] : r;
+                            return r;
+                        },
+                        [&](int q, float r) {
 #pragma unroll
-                            for (int v = 0; v < 4; ++v) {
-                                const float x = __uint_as_float(
-                                    __builtin_amdgcn_raw_buffer_load_b32(rx, arow[rb][v] + 4u * (uint32_t)k, 0, 0));
-                                acc[rb][b][v] = fmaf(x, w, acc[rb][b][v]);
-                            }
-                    }
+                            for (int i = 0; i < 4 * RB; ++i) acc[i / 4][b][i % 4] = q == i ? r : acc[i / 4][b][i % 4];
+                        },
+                        [&](int q, int k) {
+                            const int m = (q / 4) * 16 + 4 * g + q % 4;
+                            const int p = s_rows[c0 + min(m, m_valid - 1)];
+                            const uint32_t row = (uint32_t)(GATHER ? p / a.k_top : p) * (uint32_t)K * 4u;
+                            return __builtin_bit_cast(
+                                f32x4, __builtin_amdgcn_raw_buffer_load_b128(rx, row + 4u * (uint32_t)k, 0, 0));
+                        },
+                        [&](int k) {
+                            const uint32_t wo = TRANS ? (uint32_t)k * ldb2 + 4u * (uint32_t)col
+                                                      : (uint32_t)col * ldb2 + 4u * (uint32_t)k;
+                            return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rw, wo, 0, 0));
+                        });
                 }
             }
         }
