@@ -149,13 +149,28 @@ struct GemmArgs {
 };
 constexpr int kTailMaxSplit = 8;
 constexpr int kTailMinKTiles = 8;  // K tiles per tail split at least (shorter splits lose to the fixup)
-// A launch of at most half a round (all its tiles in the tail): the splits'
-// partials (256 KB each, written through and read back with every CU doing so
-// at once) cost about 25 us, 1.5 us per K tile. Qwen3 down (24 K tiles)
-// T=700 / 1000 split in two 54.6 / 58.2, whole 43.6 / 47.4 us; behind full
-// rounds, where other CUs are still computing, the split pays (T=2048 / 4096
-// 73 / 120.5 against 79.2 / 126 us).
-constexpr int kTailAloneMinKTiles = 40;
+// K parts of each of R tiles, R <= C / 2, that make up the last round of an
+// XCD's C CUs; `full` tiles ran before them. Behind full rounds, where other CUs
+// are still computing, as many as fit (Qwen3 down T=2048 / 4096 73 / 120.5 against
+// 79.2 / 126 us whole). A lone round pays for its partials itself: every part
+// writes 256 KB through and reads its share back while all the others do. It is
+// split where that spares more than kTailAloneSaves K tiles of ~1 us, and at least
+// kTailAlonePerPart of them for each 1 / C of the round's CUs that writes partials.
+// Measured over R = 1 .. 16, 16 to 64 K tiles (both GEMMs, 250 rows per expert):
+// split / whole us at R parts x K tiles spared 16 x 2 x 16 70 / 60, 12 x 2 x 16 60 /
+// 59, 8 x 3 x 16 43 / 45, 8 x 4 x 24 51 / 57, 4 x 4 x 24 38.5 / 50, 6 x 3 x 16 38 /
+// 44, 4 x 8 x 56 60 / 98; of 16 K tiles (8 spared) 31.8 / 27.2 at R = 6, 25 / 26 at 1.
+constexpr int kTailAloneSaves = 8;
+constexpr int kTailAlonePerPart = 21;
+__host__ __device__ inline int tail_parts(int R, int C, int full, int nk) {
+    if (R <= 0 || 2 * R > C) return 1;
+    int S = C / R;
+    if (S > kTailMaxSplit) S = kTailMaxSplit;
+    if (S > nk / kTailMinKTiles) S = nk / kTailMinKTiles;
+    if (S <= 1) return 1;
+    const int saves = nk - (nk + S - 1) / S;
+    return full > 0 || (saves > kTailAloneSaves && saves * C >= kTailAlonePerPart * R * S) ? S : 1;
+}
 
 // Kernel shapes (the codes of candle_moe_set_tile_policy; the missing codes
 // belonged to measured variants that are not shipped and are rejected).

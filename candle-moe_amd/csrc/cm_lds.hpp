@@ -256,12 +256,10 @@ __device__ __forceinline__ bool splitk_fixup(const GemmArgs& a, f32x16 (&acc)[MB
 }
 
 // Work item of this workgroup under tail balance (GemmArgs::tail_cus = C > 0).
-// (A launch that is all tail, full = 0, splits only from kTailAloneMinKTiles K
-// tiles on.) XCD x takes a contiguous range of nx of the `live` tiles, as xcd_logical;
+// XCD x takes a contiguous range of nx of the `live` tiles, as xcd_logical;
 // its first nx - R (R = nx mod C) tiles run whole, in nx / C full rounds over
 // the XCD's C CUs. The R tiles of the last round are split along K into
-// S = min(C / R, 8, K tiles / 8) parts when R <= C / 2, so that R * S workgroups
-// share that round instead of R. Split j of tail tile t of XCD x uses partial
+// S = tail_parts() parts, so that R * S workgroups share that round instead of R. Split j of tail tile t of XCD x uses partial
 // slot x*C + t*S + j and counter x*C + t. Returns false for a workgroup
 // without work.
 __device__ __forceinline__ bool tail_item(int live, int C, int nk_all, int& tile, int& ks, int& nsplit, int& slot0,
@@ -272,9 +270,7 @@ __device__ __forceinline__ bool tail_item(int live, int C, int nk_all, int& tile
     const int nx = per + (xcd < rem ? 1 : 0);
     const int base = xcd * per + (xcd < rem ? xcd : rem);
     const int R = nx % C, full = nx - R;
-    int S = 1;
-    if (R > 0 && 2 * R <= C && (full > 0 || nk_all >= kTailAloneMinKTiles))
-        S = min(min(C / R, kTailMaxSplit), nk_all / kTailMinKTiles);
+    const int S = tail_parts(R, C, full, nk_all);
     ks = 0;
     nsplit = 1;
     slot0 = ctr = 0;

@@ -59,3 +59,20 @@ def test_workspace_never_shrinks(H, I, E, k, dt):
         n = size(T, H, I, E, k, dt)
         assert n >= last > 0 or (T == 1 and n > 0), (T, last, n)
         last = n
+
+
+def test_tail_parts(tmp_path):
+    """K parts of the tiles of a 256x256 launch's last round (tests/cpp/tail_parts.cpp)."""
+    import os
+    import shutil
+    import subprocess
+
+    cxx = shutil.which("g++") or shutil.which("c++")
+    if cxx is None:
+        pytest.skip("no host C++ compiler")
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    exe = str(tmp_path / "tail_parts")
+    subprocess.run([cxx, "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__", "-isystem", "/opt/rocm/include",
+                    os.path.join(root, "tests", "cpp", "tail_parts.cpp"), "-o", exe], check=True)
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0 and r.stdout.strip() == "ok", r.stdout + r.stderr
