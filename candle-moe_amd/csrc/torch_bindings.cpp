@@ -96,14 +96,19 @@ bool is_index(const at::Tensor* t, const at::Device& dev, at::IntArrayRef sizes)
     return is(t, at::kInt, dev, sizes) || is(t, at::kUInt32, dev, sizes);
 }
 
-// Calls f(), releasing the interpreter lock, and returns its status.
+// The status of f(), called without the interpreter lock. f calls the C ABI only
+// (tensors are read before: they may raise, which takes the lock).
+template <class F>
+int unlocked(F&& f) {
+    struct Unlock {
+        PyThreadState* state = PyEval_SaveThread();
+        ~Unlock() { PyEval_RestoreThread(state); }
+    } unlock;
+    return f();
+}
 template <class F>
 PyObject* call(F&& f) {
-    int rc;
-    Py_BEGIN_ALLOW_THREADS
-    rc = f();
-    Py_END_ALLOW_THREADS
-    return PyLong_FromLong(rc);
+    return PyLong_FromLong(unlocked(f));
 }
 
 template <class F>
@@ -193,10 +198,10 @@ PyObject* py_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
         od.data = out.numel() ? out.data_ptr() : nullptr;
         od.strides[0] = out.stride(0);
         od.strides[1] = out.stride(1);
-        int rc;
-        Py_BEGIN_ALLOW_THREADS
-        rc = g_forward(&m, &d[0], &d[1], &d[2], has_down ? &d[3] : nullptr, &d[4], &d[5], (uint32_t)moe_type, &od, s);
-        Py_END_ALLOW_THREADS
+        const int rc = unlocked([&] {
+            return g_forward(&m, &d[0], &d[1], &d[2], has_down ? &d[3] : nullptr, &d[4], &d[5], (uint32_t)moe_type, &od,
+                             s);
+        });
         return rc == CANDLE_MOE_OK ? THPVariable_Wrap(std::move(out)) : PyLong_FromLong(rc);
     });
 }
@@ -221,9 +226,10 @@ PyObject* py_router(PyObject*, PyObject* const* a, Py_ssize_t n) {
             Py_RETURN_NONE;
         void* s;
         if (!stream_of(x, &s)) return nullptr;
+        void* p[5];
+        for (int i = 0; i < 5; ++i) p[i] = t[i]->data_ptr();
         return call([&] {
-            return g_router(x.data_ptr(), w.data_ptr(), t[2]->data_ptr(), t[3]->data_ptr(), t[4]->data_ptr(), (int)T,
-                            (int)H, (int)E, (int)k, (uint32_t)code, s);
+            return g_router(p[0], p[1], p[2], p[3], p[4], (int)T, (int)H, (int)E, (int)k, (uint32_t)code, s);
         });
     });
 }
@@ -270,14 +276,16 @@ PyObject* prepared(PyObject* const* a, Py_ssize_t n, bool fp8) {
         void* s;
         if (!stream_of(*x, &s)) return nullptr;
         const uint32_t code = (uint32_t)dtype_code(ty);
-        auto p = [](const at::Tensor* t) { return t ? t->data_ptr() : nullptr; };
-        auto f = [](const at::Tensor* t) { return t ? static_cast<const float*>(t->data_ptr()) : nullptr; };
+        const at::Tensor* all[10] = {x, gate, up, down, rw, idx, out, sc[0], sc[1], sc[2]};
+        void* p[10];
+        for (int i = 0; i < 10; ++i) p[i] = all[i] ? all[i]->data_ptr() : nullptr;
         return call([&] {
             if (fp8)
-                return g_fp8(p(x), p(gate), p(up), p(down), f(sc[0]), f(sc[1]), f(sc[2]), p(rw), p(idx), p(out), (int)T,
-                             (int)H, (int)I, (int)E, (int)k, (int)v[2], (uint32_t)v[3], code, s);
-            return g_packed(p(x), p(gate), p(up), p(down), p(rw), p(idx), p(out), (int)T, (int)H, (int)I, (int)E, (int)k,
-                            (int)v[2], (uint32_t)v[3], code, s);
+                return g_fp8(p[0], p[1], p[2], p[3], static_cast<const float*>(p[7]), static_cast<const float*>(p[8]),
+                             static_cast<const float*>(p[9]), p[4], p[5], p[6], (int)T, (int)H, (int)I, (int)E, (int)k,
+                             (int)v[2], (uint32_t)v[3], code, s);
+            return g_packed(p[0], p[1], p[2], p[3], p[4], p[5], p[6], (int)T, (int)H, (int)I, (int)E, (int)k, (int)v[2],
+                            (uint32_t)v[3], code, s);
         });
     });
 }

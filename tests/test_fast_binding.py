@@ -188,3 +188,38 @@ def test_stream(fast):
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, want)
+
+
+def _calls():
+    """Every entry point with its tensors, small and valid."""
+    T, H, I, E, k = 3, 64, 64, 4, 2
+    bf = dict(dtype=torch.bfloat16, device="cuda")
+    f32, i32 = dict(device="cuda"), dict(dtype=torch.int32, device="cuda")
+    w, idx, te = torch.full((T, k), 0.5, **f32), torch.zeros(T, k, **i32), torch.zeros(T, k, **i32)
+    x, out, G = torch.ones(T, H, **bf), torch.zeros(T, H, **bf), torch.ones(E, H, I, **bf)
+    u8 = dict(dtype=torch.uint8, device="cuda")
+    q, sc = torch.zeros(E, I, H, **u8), torch.ones(E, I, **f32)
+    moe = cm.FusedMoE.new(E, k, cm.Activation.Silu)
+    return {
+        "topk": (cm.apply_topk_softmax_inplace, [torch.zeros(T, E, **f32), w, idx, te], ()),
+        "router": (cm.router_topk, [x, torch.ones(E, H, **bf), w, idx, te], ()),
+        "forward": (lambda *a: moe.forward(*a, 0), [x, G, G.clone(), G.clone(), w, idx], ()),
+        "packed": (cm.fused_moe_packed, [x, G, G.clone(), G.clone(), w, idx, out], (E, k, 0, 0)),
+        "fp8": (cm.fused_moe_fp8, [x, q, q.clone(), q.clone(), sc, sc.clone(), sc.clone(), w, idx, out], (E, k, 0, 0)),
+    }
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["topk", "router", "forward", "packed", "fp8"])
+def test_tensor_that_refuses_its_pointer(name):
+    """A tensor whose data pointer must not be read raises, as on the ctypes
+    route, whichever argument it is; the interpreter lock is held by then."""
+    for i in range(len(_calls()[name][1])):
+        fn, tensors, rest = _calls()[name]
+        tensors[i] = tensors[i].clone()
+        torch._C._set_throw_on_mutable_data_ptr(tensors[i])
+        with pytest.raises(RuntimeError, match="data pointer"):
+            fn(*tensors, *rest)
+    fn, tensors, rest = _calls()[name]
+    fn(*tensors, *rest)
+    torch.cuda.synchronize()
