@@ -18,6 +18,7 @@ from __future__ import annotations
 import ctypes
 import enum
 import os
+import sys
 from typing import Optional, Sequence
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -77,8 +78,11 @@ class CmFusedMoE(ctypes.Structure):
 _lib = None
 # candle_moe._fast bound to _lib (csrc/torch_bindings.cpp), or None before the
 # library is loaded and where the module is not built: the calls below then
-# describe their tensors here.
+# describe their tensors here. Bound once torch has been imported (by whoever
+# makes the tensors): a program that only uses the C entry points need not wait
+# for that import.
 _native = None
+_native_tried = False
 
 
 def _bind_native(L: ctypes.CDLL):
@@ -99,7 +103,7 @@ def _bind_native(L: ctypes.CDLL):
 
 def lib() -> ctypes.CDLL:
     """The loaded HIP library (raises if it has not been built)."""
-    global _lib, _native
+    global _lib, _native, _native_tried
     if _lib is None:
         if not os.path.exists(LIB_PATH):
             raise RuntimeError(
@@ -176,8 +180,10 @@ def lib() -> ctypes.CDLL:
         L.candle_moe_fused_moe_forward.restype = i32
         L.candle_moe_validate_fused_moe.argtypes = [mp, tp, tp, tp, tp, tp, tp, u32, tp]
         L.candle_moe_validate_fused_moe.restype = i32
-        _native = _bind_native(L)
         _lib = L
+    if not _native_tried and "torch" in sys.modules:
+        _native_tried = True
+        _native = _bind_native(_lib)
     return _lib
 
 

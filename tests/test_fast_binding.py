@@ -1,6 +1,7 @@
 """candle_moe._fast against the ctypes route: the same descriptors, results and
 errors for every form of tensor the entry points take or refuse."""
 import ctypes
+import os
 
 import pytest
 import torch
@@ -223,3 +224,16 @@ def test_tensor_that_refuses_its_pointer(name):
     fn, tensors, rest = _calls()[name]
     fn(*tensors, *rest)
     torch.cuda.synchronize()
+
+
+def test_the_library_loads_without_torch():
+    """lib() alone does not import torch; the binding follows once it is there."""
+    import subprocess
+    import sys
+
+    code = ("import sys, candle_moe as cm; cm.lib(); cm.lib(); assert 'torch' not in sys.modules; "
+            "assert cm._native is None; import torch; cm.lib(); "
+            "import importlib.util as u; "
+            "assert (cm._native is not None) == (u.find_spec('candle_moe._fast') is not None)")
+    subprocess.run([sys.executable, "-c", code], check=True, timeout=300,
+                   env=dict(os.environ, PYTHONPATH=os.path.dirname(os.path.dirname(cm.__file__))))
