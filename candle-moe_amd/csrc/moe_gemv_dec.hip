@@ -66,9 +66,9 @@ constexpr int kDvStep = 32;  // K per step (one MFMA deep)
 // steps in flight per wave: 4, or 2 for 6 or 8 columns per lane, so that a
 // wave stays within 256 registers and two workgroups share a CU; halved where
 // each column takes WCH = 2 chunks of 16 bytes per step (the same bytes in
-// flight). f32: twice the bytes per weight, so 2 steps from 3 columns on.
+// flight). f32 (4 columns): twice the bytes per weight, so 2 steps.
 template <int CPL, int WCH = 1, bool F32 = false>
-constexpr int dec_ring() { return F32 ? (CPL >= 3 ? 2 : 4) : (CPL >= 6 ? 2 : 4) / WCH; }
+constexpr int dec_ring() { return F32 ? 2 : (CPL >= 6 ? 2 : 4) / WCH; }
 
 // Operand j of a transposed 8 x CPL block: r[t] holds k-row t of CPL
 // consecutive columns (pairs of 16-bit values, low half first); the result
@@ -311,7 +311,7 @@ __global__ __launch_bounds__(64 * kDvWaves, 2) void moe_dec_gemv(DecArgs a) {
     // form (whose v_perm transpose the pairwise conversion replaces); [N,K]:
     // two 16-byte chunks of 4 k, 128 contiguous bytes per column and step.
     constexpr bool F32 = DT == kF32;
-    static_assert(!F32 || (!W8 && !PK && CPL <= 4), "f32: API layout, at most 4 columns per lane");
+    static_assert(!F32 || (!W8 && !PK && CPL == 4), "f32: API layout, 4 columns per lane");
     constexpr int WCH = (W8 || MODE == kFc2Rows) ? 2 : 1;
     constexpr int KSTEP = F32 ? kDvStep : (W8 ? 64 : kDvStep) * WCH;
     constexpr int KG = F32 ? 8 : (W8 ? 16 : 8) * WCH;  // k per lane group per step
@@ -811,13 +811,7 @@ template <int DT, int MODE>
 hipError_t launch_mode(const DecArgs& a, hipStream_t stream) {
     const bool rb2 = a.rows_max > 16;
     if constexpr (DT == kF32) {
-        // f32: 4 columns per lane ([N,K] also 3 and 2)
-        if (a.w8 || a.packed) return hipErrorInvalidValue;
-        if constexpr (MODE == kFc2Rows) {
-            if (a.cpl == 2) return rb2 ? launch_cfg<DT, MODE, 2, 2>(a, stream) : launch_cfg<DT, MODE, 1, 2>(a, stream);
-            if (a.cpl == 3) return rb2 ? launch_cfg<DT, MODE, 2, 3>(a, stream) : launch_cfg<DT, MODE, 1, 3>(a, stream);
-        }
-        if (a.cpl != 4) return hipErrorInvalidValue;
+        if (a.w8 || a.packed || a.cpl != 4) return hipErrorInvalidValue;
         return rb2 ? launch_cfg<DT, MODE, 2, 4>(a, stream) : launch_cfg<DT, MODE, 1, 4>(a, stream);
     } else {
     if (a.cpl == 2) return rb2 ? launch_cfg<DT, MODE, 2, 2>(a, stream) : launch_cfg<DT, MODE, 1, 2>(a, stream);
