@@ -1239,10 +1239,13 @@ size_t router_ws_bytes(int T, int H, int E, int dtype) {
     return ks > 1 ? (size_t)ks * T * E * sizeof(float) : 0;
 }
 size_t router_upto_bytes(int T, int H, int E, int dtype) {
-    size_t most = router_ws_bytes(T, H, E, dtype);
-    for (int t = 32; t < T + 32 && t <= kRouterSplitTokens; t += 32)  // (the most tokens of each tile count)
-        most = std::max(most, router_ws_bytes(std::min(t, T), H, E, dtype));
-    return most;
+    if (dtype == kF32 || E <= 32 || E > 128) return 0;
+    // (splits * tokens of a small batch: at most kRouterMaxSlots splits, 64
+    // workgroups of 32 tokens; every call's host time)
+    const int most = std::min(kRouterMaxSlots, (H + 63) / 64 / 2);
+    if (most < 2) return 0;
+    const size_t small = (size_t)std::min(most * std::min(T, kRouterSplitTokens), 64 * 32) * E * sizeof(float);
+    return T > kRouterSplitTokens ? std::max(small, router_ws_bytes(T, H, E, dtype)) : small;
 }
 
 template <int DT, int NB>
