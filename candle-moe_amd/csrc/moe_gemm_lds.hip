@@ -39,7 +39,11 @@ using namespace lds;
 // over the waves: wave (wm, wn) multiplies it with NB / 2 of the NB column
 // blocks it reads anyway (those from index wm * NB / 2), one more A fragment
 // and NB / 2 more MFMAs per k16 step. The K loop exists twice, with and without
-// the block, chosen per tile; the block's rows are stored directly.
+// the block, chosen per tile (an instance without extended tiles takes as long:
+// exactly 128 rows per expert, Qwen3 T=512 98.2 us before, 91.3 with the second
+// loop in it, Qwen3-30B-A3B T=2048 / 4096 on 128x256 286.1 / 440.3, 286.1 / 440.9).
+// The block's rows leave with the tile's in the staged epilogue; in the
+// accumulating expert-set mode they are added directly.
 // Measured (gate/up / down): Qwen3 T=500 on 128x128 tiles 97 / 46 -> 66 / 32
 // us, Qwen3-30B-A3B T=2000 / 4096 on 128x256 tiles 212 / 110 -> 184 / 98 and 298
 // / 165 -> 283 / 158 us. Not on the 256x256 kernel: its extended tiles took 13 %
