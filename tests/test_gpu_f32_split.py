@@ -57,7 +57,7 @@ def test_f32_split_accuracy(tile, T, H, I, E, k, mt):
 @pytest.mark.parametrize("mt", [O.QWEN3, O.NOMIC])
 def test_f32_split_non_finite_and_extreme_inputs(tile, mt):
     # an infinity, a NaN, a value whose bf16 part would round to infinity and
-    # values whose low parts are subnormal: what f32 FMAs give. (ReLU: an
+    # values whose low parts would be subnormal unscaled: what f32 FMAs give. (ReLU: an
     # infinite pre-activation stays infinite or becomes zero.)
     T, H, I, E, k = 40, 64, 72, 2, 1
     x, G, U, D, rw, ri = moe_inputs(T, H, I, E, k, O.F32, 950, mt)

@@ -1,6 +1,6 @@
-"""router_topk past 256 tokens: K splits over workgroups where they pay, one pass
-otherwise and under graph capture; stages of two K tiles
-with odd tile counts and K tails. Inputs whose sums are exact in f32 (small
+"""router_topk past 256 tokens: K splits over workgroups where they pay, the same
+sums inside one workgroup per tile under graph capture, one pass otherwise; stages
+of two K tiles with odd tile counts and K tails. Inputs whose sums are exact in f32 (small
 integers over powers of two), so every form gives the oracle's indices bit for
 bit and its weights within 1e-6 (f32 exp and quotient, as in
 tests/test_gpu_router.py)."""
