@@ -356,14 +356,17 @@ static void choose_dec_slices(Problem& p) {
     // its items would leave CUs idle (Nomic's fc2 has 96 of them)
     const int cols = p.dtype == kF32 ? 64 : 128;
     const double part = p.dtype == kF32 ? kDecPartBytesF32 : kDecPartBytes;
-    // 16-bit also where the GEMM's 64-column blocks are few (a quarter of
-    // the CUs) and stream 1 MiB each: one or two tokens over large experts.
-    // Steps unsliced / sliced: Qwen3 T=1 36.0 / 27.8 us (pre-packed 38.0 /
+    // Also where the GEMM's 64-column blocks are few (a quarter of the CUs) and
+    // stream 1 MiB each, f32 ones 512 KiB: one or two tokens over large experts,
+    // or few experts. f32, unsliced / sliced (the 32-row tiles): H 4096 I 1536 E 1
+    // k 1 T=1 / 32 66.8 / 88.3 against 32.7 / 42.1 (55 / 58), E 2 T=64 162 against
+    // 69.9 (116), H 1024 I 512 E 8 k 2 T=64 34.7 against 32.6 (44.5).
+    // 16-bit, unsliced / sliced: Qwen3 T=1 36.0 / 27.8 us (pre-packed 38.0 /
     // 34.3), H 8192 I 2048 k 1 T=1 85.6 / 37.9, H 4096 I 512 E 128 k 8 T=1
     // 51.0 / 32.2. At 96 blocks (Qwen3 T=2) 57.9 / 43.0, but pre-packed,
     // which takes the same slices to give the same bits, 48.2 / 51.1.
-    const bool few = p.dtype != kF32 && !p.fp8 && groups * cdiv(p.I, 64) <= 64 &&
-                     (long long)(q3 ? 2 : 1) * p.H * 128 >= (1 << 20);
+    const bool few = !p.fp8 && groups * cdiv(p.I, 64) <= 64 &&
+                     (long long)(q3 ? 2 : 1) * p.H * 64 * (p.dtype == kF32 ? 4 : 2) >= (p.dtype == kF32 ? 1 << 19 : 1 << 20);
     if (groups * cdiv(p.I, cols) < 256 && (wbytes >= kDecSliceBytes || few))
         p.dec_ks1 = dec_slices(P, p.I, p.H, q3 ? 2 : 4, q3 ? 2 : 1, part);
     if (p.dtype == kF32 && groups * cdiv(p.H, cols) < 256) p.dec_ks2 = dec_slices(P, p.H, p.I, 4, 1, part);
