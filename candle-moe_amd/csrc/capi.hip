@@ -531,7 +531,11 @@ static int check_problem(int T, int H, int I, int E, int k, int act, uint32_t mo
             p.cfg = kLds128;
         // (kOneTileRows .. kTwoTileRows rows: one 256-row tile per expert
         // against two of 128: Qwen3-30B-A3B T=2600 / 3000 400 / 420 against 372
-        // / 382 us on 256x256; T=4096, 256 rows: 486 against 505 us)
+        // / 382 us on 256x256; T=4096, 256 rows: 486 against 505 us. Lines for
+        // near-uniform routing, which is all the host can assume: with Zipf(0.7)
+        // and Zipf(1.2) router biases 128x256 leads at 184 rows too, Qwen3-30B-A3B
+        // 437 / 448 against 472 / 466, H 2048 I 768 E 64 k 4 228 / 252 against 262 /
+        // 254 us, while uniform batches take 411 against 367 and 228 against 228)
         else if (H <= 2048 && P < 1024 * touched && P >= kTwoTileRows * touched &&
                  (long long)cdiv(H, 256) * est_tiles(128) >= 2 * dev_wgs)
             p.cfg = kLds128x256o2;
