@@ -1273,7 +1273,8 @@ int fused_moe_impl(const void* x, const void* gate, const void* up, const void* 
     const bool served = slot >= 0 && T <= w->served[slot].T;
     const size_t full = served ? L.total : upto_bytes(p);
     w = owned_ws_locked(dev, s, L.total, full, e);
-    if (w && !served && w->bytes >= full) {
+    // (without memory for the reserve: not asked for again in every call)
+    if (w && !served && (w->bytes >= full || !is_capturing(s))) {
         if (slot < 0) slot = w->next++ & 3;
         std::copy(layer, layer + 8, w->served[slot].layer);
         w->served[slot].T = T;
